@@ -116,6 +116,9 @@ struct RenderParams {
   const float* records;       // [P][32]
   const float* colors;        // [P][C] colour path; [P][cstride] per-splat features (mix)
   uint32_t* tile_order;       // [tiles] launch order, written by launch_render
+  uint32_t parts;             // workgroups per tile the grid levels are dealt over (1, 2, 4 or 8), set by launch_render
+  uint32_t parts_log2;
+  uint32_t part_levels;       // levels of a part (the most any has)
   float* out_color;
   float* out_others;
   float* final_T;

@@ -10,22 +10,32 @@
 // kMix instantiations.
 //
 // Layout: one 256-thread workgroup per 16x16 tile, one lane per pixel (four
-// 64-lane waves of 16x4 pixels).  The tile's sorted splats are staged in LDS
-// in batches of 256 packed 128-byte records (structure-of-arrays float4
-// chunks, so a wave reads a record with broadcast ds_read_b128).  Workgroups
-// launch heaviest tile first (tile_order_kernel), dealt over the XCDs in runs
-// of 16.
+// 64-lane waves of 16x4 pixels); frames of few tiles deal the grid's levels
+// over several workgroups per tile (level_parts).  The tile's sorted
+// splats are staged in LDS in batches of 256 packed 128-byte records
+// (structure-of-arrays float4 chunks).  Workgroups launch heaviest tile first
+// (tile_order_kernel), dealt over the XCDs in runs of 16.
 //
-// Work split inside a wave:
-//  - compositing runs splat by splat for all 64 pixels: a whole-wave skip when
-//    the wave's pixel block is outside the splat's acceptance bbox, a per-lane
-//    rcp-based early reject, then the exact test;
-//  - an accepted hit updates the depth/normal/distortion state at once and
-//    enqueues (grid coordinate, weight, level count) in a per-lane LDS queue;
+// Work split inside a wave, per batch:
+//  - test pass: the splats whose acceptance bbox meets the wave's pixel block
+//    (one bit per splat, balloted by the lanes that stage them) one after the
+//    other for all 64 pixels: a conservative rcp-based test, whose survivors
+//    go to a per-lane LDS list;
+//  - hit pass: each lane works through its own list, in order, at its own
+//    splats: the exact test, the depth/normal/distortion state, and
+//    (grid coordinate, weight, level count) into a per-lane LDS queue;
 //  - when any lane's queue is full the wave drains: up to 64 pending hits,
 //    oldest first, are spread one per lane whatever pixel they belong to, so
 //    the gathers and the interpolation run with all lanes busy; each pixel's
 //    lane then accumulates its own hits in front-to-back order.
+//
+// A splat reaches ~2.8 pixels of a wave's block that its bbox meets, so the
+// exact test and the blending, run splat by splat, had 61 of 64 lanes idle;
+// lists bring that to one pass per ~30 hits.  Compositing alone (no hit
+// enqueued), ms before / after: 4M splats at 1920x1080 14.2 / 7.0, 1M splats
+// at 1600x1064 1.45 / 1.06; whole render, same order: 40.2 / 34.1, 6.13 / 5.93
+// (bound by the drains' lookups); 400k SH-coloured splats at 1237x822 1.21 /
+// 0.80; 2,000 splats at 128x128 0.285 / 0.183 and 0.125 with level parts.
 #include <type_traits>
 
 #include "hashgrid.h"
@@ -45,9 +55,20 @@ namespace nest {
 // drain keeps only ~47 of 64 lanes busy.
 constexpr int kRenderThreads = 256;
 constexpr int kBatch = 256;    // splats staged in LDS per batch
-constexpr int kRecChunks = 8;  // float4 chunks of the record staged per splat
+constexpr int kRecChunks = 7;  // float4 chunks of the record staged per splat (the bbox, chunk 7, stays in registers)
 constexpr int kQueue = 4;      // pending hash lookups per pixel
+constexpr int kList = 8;       // candidate splats a pixel holds between the test and the hit pass
 constexpr int kWaveLanes = 64;
+constexpr int kWaves = kRenderThreads / kWaveLanes;
+
+// A wave's pixel block: 16 x 4 pixels, four lanes to a 2 x 2 quad.  (8 x 8
+// blocks skip more splats but leave a quad's and a wave's lookups on more
+// lines: on the 1M-splat frame 6.17-6.20 ms against 5.97-6.00, on the
+// 400k-splat colour frame 0.77 against 0.80; rows of 16 lanes instead of
+// quads 6.03 and, on the 4M-splat frame, 34.9 against 34.1.)
+constexpr uint32_t kBlockW = 16, kBlockH = 4;
+__device__ __forceinline__ uint32_t lane_x(uint32_t l) { return (l & 1u) | ((l >> 1) & 14u); }
+__device__ __forceinline__ uint32_t lane_y(uint32_t l) { return ((l >> 1) & 1u) | ((l >> 4) & 2u); }
 
 __device__ __forceinline__ uint64_t lanemask_lt64() {
   const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
@@ -143,9 +164,11 @@ __device__ __forceinline__ void drain_round(const GridParams& g, nest_i32x4 rsrc
 // Levels at or past a hit's level count give 0, and fmaf(0, w, acc) == acc
 // (w is finite and the accumulators never hold -0), as in the round drain.
 // isrc is this wave's 64-byte table of moved hits: owner lane | slot << 6,
-// indexed by the taking lane's rank among the empty lanes.
+// indexed by the taking lane's rank among the empty lanes.  Output level l is
+// grid level first + l * lstep (level parts; structured grids only).
 template <int F, int NACC, bool kHalf, bool kStructured>
-__device__ __forceinline__ void drain_compact(const GridParams& g, nest_i32x4 rsrc, float4 (*hq)[kRenderThreads],
+__device__ __forceinline__ void drain_compact(const GridParams& g, uint32_t first, uint32_t lstep, nest_i32x4 rsrc,
+                                              float4 (*hq)[kRenderThreads],
                                               uint8_t (*hl)[kRenderThreads], uint8_t* isrc, int& qhead, int& qn,
                                               float* acc) {
   static_assert(F <= 4, "a level's values fit one queue slot");
@@ -197,7 +220,7 @@ __device__ __forceinline__ void drain_compact(const GridParams& g, nest_i32x4 rs
   // level l is interpolated (its load registers are free then), so they are
   // in flight during level l's hand-off through LDS and the owners' sums.
   constexpr int kLevels = NACC / F;
-  const LevelQuadPtr lqb = (LevelQuadPtr)g.lq;
+  const LevelQuadPtr lqb = (LevelQuadPtr)g.lq + first;
   LevelCorners cn;
   float vals[8][F];
   bool look = work && 0u < nlev;
@@ -206,12 +229,12 @@ __device__ __forceinline__ void drain_compact(const GridParams& g, nest_i32x4 rs
   if (look) {
     level_fetch<F, kHalf, kStructured>(g, rec, 0, u, rsrc, cn, vals);
   }
-  if constexpr (kStructured) rec_next = level_record(lqb, 1);
+  if constexpr (kStructured) rec_next = level_record(lqb, (int)lstep);
 #pragma unroll
   for (int l = 0; l < kLevels; l++) {
     nest_u32x4 rec_after = {0u, 0u, 0u, 0u};
     if constexpr (kStructured)
-      if (l + 2 < kLevels) rec_after = level_record(lqb, l + 2);
+      if (l + 2 < kLevels) rec_after = level_record(lqb, (l + 2) * (int)lstep);
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (look) corners_sum_r<F, kHalf>(cn, vals, v);
     bool next = false;
@@ -464,8 +487,26 @@ __device__ __forceinline__ float kernel_g(int kt, float rho, float shape) {
   return expf_ref(power);
 }
 
-__device__ __forceinline__ bool splat_hit(float4 q0, float4 q1, float4 q2, float cut, float pxf, float pyf, float beta,
-                                          SplatHit& h, int kt = 0, const float& shape = 0.0f) {
+// Conservative form of the test below, for the pass that lists a pixel's
+// candidates: an rcp-based rho3d within 1e-6 of the exact one, scaled down by
+// 1e-5, above the splat's cut and rho2d above it too means alpha < 1/255 in
+// the exact test.  False only for such pairs; NaNs are candidates.
+__device__ __forceinline__ bool splat_near(float4 q0, float4 q1, float4 q2, float cut, float pxf, float pyf) {
+  const float Tu0 = q0.x, Tu1 = q0.y, Tu2 = q0.z, Tv0 = q0.w;
+  const float Tv1 = q1.x, Tv2 = q1.y, Tw0 = q1.z, Tw1 = q1.w;
+  const float Tw2 = q2.x;
+  const float k0 = pxf * Tw0 - Tu0, k1 = pxf * Tw1 - Tu1, k2 = pxf * Tw2 - Tu2;
+  const float l0 = pyf * Tw0 - Tv0, l1 = pyf * Tw1 - Tv1, l2 = pyf * Tw2 - Tv2;
+  const float p0 = k1 * l2 - k2 * l1, p1 = k2 * l0 - k0 * l2, p2 = k0 * l1 - k1 * l0;
+  const float dx = q2.y - pxf, dy = q2.z - pyf;
+  const float rho2d = 2.0f * (dx * dx + dy * dy);
+  const float rc = __builtin_amdgcn_rcpf(p2);
+  const float sxa = p0 * rc, sya = p1 * rc;
+  return !((sxa * sxa + sya * sya) * 0.99999f > cut && rho2d > cut);
+}
+
+__device__ __forceinline__ bool splat_hit(float4 q0, float4 q1, float4 q2, float pxf, float pyf, float beta,
+                                          SplatHit& h, int kt = 0, float shape = 0.0f) {
   const float Tu0 = q0.x, Tu1 = q0.y, Tu2 = q0.z, Tv0 = q0.w;
   const float Tv1 = q1.x, Tv2 = q1.y, Tw0 = q1.z, Tw1 = q1.w;
   const float Tw2 = q2.x;
@@ -475,14 +516,6 @@ __device__ __forceinline__ bool splat_hit(float4 q0, float4 q1, float4 q2, float
   if (p2 == 0.0f) return false;
   const float dx = q2.y - pxf, dy = q2.z - pyf;
   const float rho2d = 2.0f * (dx * dx + dy * dy);
-  // Per-lane early reject: an rcp-based rho3d within 1e-6 of the exact one,
-  // scaled down by 1e-5, above the splat's cut and rho2d above it too means
-  // alpha < 1/255 in the exact test.  NaNs take the exact path.
-  {
-    const float rc = __builtin_amdgcn_rcpf(p2);
-    const float sxa = p0 * rc, sya = p1 * rc;
-    if ((sxa * sxa + sya * sya) * 0.99999f > cut && rho2d > cut) return false;
-  }
   const float sx = p0 / p2, sy = p1 / p2;
   const float rho3d = sx * sx + sy * sy;
   const float rho = fminf(rho3d, rho2d);
@@ -555,14 +588,34 @@ __device__ __forceinline__ uint8_t hit_levels(bool oob, uint32_t ap, uint32_t L)
   return (uint8_t)(max_level < 255u ? max_level : 255u);
 }
 
-// State of an accepted hit between the per-lane test and the converged
-// feature block of the render modes 4 and 13.
-struct PendingHit {
-  bool on = false;
-  float w = 0.0f, T = 0.0f;
-  SplatHit hit{};
+// Four floats of a feature row, which starts at any float.
+struct __attribute__((packed, aligned(4))) RowFloat4 {
+  float v[4];
 };
-struct NoPendingHit {};
+
+// acc[c] += w * row[c] (times the row's weight with wcoarse) for the channels
+// below the lane's ndirect; rows are p.cstride floats, read four at a time.
+template <int NACC>
+__device__ __forceinline__ void row_accumulate(const RenderParams& p, const float* row, int ndirect, float wt, float w,
+                                               float* acc) {
+#pragma unroll
+  for (int c0 = 0; c0 < NACC; c0 += 4) {
+    if (c0 < ndirect) {
+      float rv[4];
+      if (c0 + 4 <= p.cstride) {
+        const RowFloat4 r = *reinterpret_cast<const RowFloat4*>(row + c0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) rv[i] = r.v[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) rv[i] = c0 + i < ndirect ? row[c0 + i] : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (c0 + i < ndirect) acc[c0 + i] = fmaf(p.wcoarse ? rv[i] * wt : rv[i], w, acc[c0 + i]);
+    }
+  }
+}
 
 // Appearance-level colour of a hit (CR/forward.cu:1945-1957): its first two
 // channels; the third only ever adds 0 * w.
@@ -710,28 +763,41 @@ template <int F, int NACC, bool kHash, bool kHalf, bool kStructured = false, int
           int kHsh = 0>
 __global__ void __launch_bounds__(kRenderThreads) __attribute__((amdgpu_waves_per_eu(3, 8)))
 render_kernel(const RenderParams p) {
+  constexpr bool kParts = kHash && kMix == 0 && kStructured && F <= 4;  // grid levels may be split over workgroups
   __shared__ float4 srec[kRecChunks][kBatch];
   __shared__ float4 hq[kHash ? kQueue : 1][kRenderThreads];
-  __shared__ uint8_t hl[kHash && !kMix ? kQueue : 1][kRenderThreads];
+  __shared__ uint8_t hl[kHash && !kMix ? kQueue : 1][kHash && !kMix ? kRenderThreads : 1];
   __shared__ uint32_t hm[kMix ? kQueue : 1][kMix ? kRenderThreads : 1];
   __shared__ uint8_t isrc[kHash ? kRenderThreads : 1];  // compacted-drain item tables, 64 per wave
+  __shared__ uint8_t hlist[kList][kRenderThreads];      // candidate splats per pixel, batch indices
+  __shared__ uint64_t smask[kWaves][kWaves];            // [pixel block][64 splats] splats whose bbox meets the block
 
-  const uint32_t tile = p.tile_order[blockIdx.x];
+  // Level parts (level_parts): workgroup b runs on XCD x = b % 8, which keeps to
+  // part x % parts, the levels congruent to it.  The 8 / parts XCDs of a part
+  // share the order's tiles, XCD y of them those dealt to y, y + 8 / parts, ...
+  uint32_t pos = blockIdx.x, part = 0u;
+  if constexpr (kParts) {
+    if (p.parts > 1u) {
+      const uint32_t x = blockIdx.x % 8u, q = blockIdx.x / 8u;
+      part = x % p.parts;
+      pos = 8u * (q >> p.parts_log2) + x / p.parts + (8u >> p.parts_log2) * (q % p.parts);
+      if (pos >= p.ntiles) return;
+    }
+  }
+  const uint32_t tile = p.tile_order[pos];
   const uint32_t tx = tile % p.gx, ty = tile / p.gx;
-  const uint32_t px = tx * kTile + (threadIdx.x & 15u);
-  const uint32_t py = ty * kTile + (threadIdx.x >> 4);
+  const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveLanes);
+  const uint32_t wlane = threadIdx.x & (kWaveLanes - 1);
+  const uint32_t px = tx * kTile + lane_x(wlane);
+  const uint32_t py = ty * kTile + wid * kBlockH + lane_y(wlane);
   const bool inside = px < (uint32_t)p.W && py < (uint32_t)p.H;
   const float pxf = (float)px, pyf = (float)py;
   bool done = !inside;
-  // pixel block of this wave: 16 columns x 4 rows
-  const uint32_t wid = threadIdx.x / kWaveLanes;
-  const float wx0 = (float)(tx * kTile), wx1 = wx0 + 15.0f;
-  const float wy0 = (float)(ty * kTile + 4u * wid), wy1 = wy0 + 3.0f;
 
   const uint2 range = reinterpret_cast<const uint2*>(p.ranges)[tile];
 
   float T = 1.0f;
-  uint32_t contributor = 0, last_contributor = 0, render_number = 0;
+  uint32_t last_contributor = 0, render_number = 0;
   float acc[NACC];
 #pragma unroll
   for (int c = 0; c < NACC; c++) acc[c] = 0.0f;
@@ -745,210 +811,208 @@ render_kernel(const RenderParams p) {
   nest_i32x4 rsrc{};
   if constexpr (kHash) rsrc = table_rsrc_rows<F, kHalf>(g.table, g.table_rows);
   int qn = 0, qhead = 0;  // per-lane ring buffer of pending lookups
-  // kMix: an accepted hit's feature part waits for the converged block after
-  // the per-lane test
-  [[maybe_unused]] std::conditional_t<(kMix != 0), PendingHit, NoPendingHit> ph;
 
-  // Batches of 256 splats.  The splat index j is uniform across the wave;
-  // lanes that are done skip the body, as the reference's per-lane loop
-  // stops.  The wave pauses at a splat after which some lane's queue is full
-  // and drains, and the last pass (no splats left, or every pixel of the tile
-  // done) drains what remains, so the drain has a single call site.
+  // Batches of 256 splats, each in rounds of two passes per wave:
+  //  - test: the batch's splats whose acceptance bbox meets the wave's pixel
+  //    block (masks balloted while staging) one after the other, every lane
+  //    one pixel; a lane lists the splats that may reach it;
+  //  - hits: every lane takes its own list, in order, whatever splats the
+  //    others are at: the exact test, the blending state and the feature
+  //    lookup's queue.
+  // A round ends when some lane's list is full or the batch is through; lanes
+  // that are done list nothing, as the reference's per-lane loop stops.  The
+  // last pass (no splats left, or every pixel of the tile done) drains what
+  // the queues still hold, so the drain has a single call site.
   uint32_t start = range.x;
   for (;;) {
     const bool all_done = __syncthreads_count(done) == kRenderThreads;
     const bool last = start >= range.y || all_done;
-    uint32_t n = 0;
+    uint32_t chunk = last ? (uint32_t)kWaves : 0u;
     if (!last) {
       const uint32_t e = start + threadIdx.x;
-      if (e < range.y) {
+      const bool in = e < range.y;
+      float4 bb = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (in) {
         const uint32_t id = p.point_list[e];
         const float4* rec = reinterpret_cast<const float4*>(p.records) + 8 * (size_t)id;
 #pragma unroll
         for (int c = 0; c < kRecChunks; c++) srec[c][threadIdx.x] = rec[c];
         srec[6][threadIdx.x].w = __uint_as_float(id);  // the depth's slot: the render recomputes depth per hit
+        bb = rec[7];
+      }
+      // Splats outside a wave's pixel block: the alpha test rejects every pixel of it.
+      const float bx0 = (float)(tx * kTile), bx1 = bx0 + (float)(kBlockW - 1);
+#pragma unroll
+      for (int b = 0; b < kWaves; b++) {
+        const float by0 = (float)(ty * kTile + b * kBlockH), by1 = by0 + (float)(kBlockH - 1);
+        const uint64_t m = __ballot(in && !(bb.y < bx0 || bb.x > bx1 || bb.w < by0 || bb.z > by1));
+        if (wlane == 0u) smask[b][wid] = m;
       }
       __syncthreads();
-      n = min((uint32_t)kBatch, range.y - start);
     }
-    uint32_t j = 0;
+    const uint32_t base = start - range.x;
+    uint64_t todo = 0ull;  // splats of the current 64 still to be tested
+    uint32_t j0 = 0u;      // their first index
     for (;;) {
-    while (j < n) {
-      if constexpr (kMix) ph.on = false;
-      if (!done) {
-      contributor++;
-      do {
-        // Whole-wave skip: the wave's pixel block lies outside the splat's
-        // acceptance bbox, so the alpha test rejects every pixel of it.
-        const float4 bb = srec[7][j];
-        if (bb.y < wx0 || bb.x > wx1 || bb.w < wy0 || bb.z > wy1) break;
-        SplatHit hit;
-        if (!splat_hit(srec[0][j], srec[1][j], srec[2][j], srec[6][j].y, pxf, pyf, p.beta, hit,
-                       kKT ? p.kernel_type : 0, srec[6][j].z))
-          break;
-        const float test_T = T * (1 - hit.alpha);
-        if (test_T < 0.0001f) {
-          done = true;
-          break;
+      uint32_t cnt = 0u, pos = 0u;
+      for (;;) {
+        if (todo == 0ull) {
+          if (chunk == (uint32_t)kWaves) break;
+          const uint64_t m = smask[wid][chunk];
+          todo = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)m) |
+                 (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(m >> 32)) << 32;
+          j0 = chunk++ * kWaveLanes;
+          continue;
         }
-        const float w = hit.alpha * T;
-        render_number++;
-        if (p.max_intersections > 0 && render_number >= p.max_intersections) done = true;
-
-        const float4 q3 = srec[3][j];
-        const float depth = hit.depth;
-        const float Aa = 1 - T;
-        const float m = mfac * (1 - 0.2f / depth);
-        distortion += (m * m * Aa + M2 - 2 * m * M1) * w;
-        D += depth * w;
-        M1 += m * w;
-        M2 += m * m * w;
-        if (T > 0.5f) {
-          median_depth = depth;
-          median_contributor = (float)contributor;
-        }
-        N0 += q3.x * w;
-        N1 += q3.y * w;
-        N2 += q3.z * w;
-
-        if constexpr (kMix) {
-          ph.on = true;
-          ph.w = w;
-          ph.T = test_T;
-          ph.hit = hit;
-          break;
-        }
-        if constexpr (kHsh != 0) {
-          float xyz[3];
-          hit_world(srec[4][j], srec[5][j], srec[6][j], hit, xyz);
-          pos_x += w * xyz[0];
-          pos_y += w * xyz[1];
-          pos_z += w * xyz[2];
-          const uint32_t ap = __float_as_uint(q3.w);
-          const uint32_t id = __float_as_uint(srec[6][j].w);
-          const float* row = p.colors + (size_t)id * (uint32_t)p.cstride;
-          if constexpr (kHsh == 1 || kHsh == 5) {
-            surface_accumulate<kHsh, NACC>(p, xyz, ap, q3, row, w, acc);
-          } else {
-            float h[3];
-            if (p.hsh_dec != 1)
-              hsh_query(g, xyz, ap, h);
-            else
-              h[0] = h[1] = h[2] = 0.0f;
-            hsh_accumulate<kHsh, NACC>(p, row, h, w, acc);
-          }
-          appearance_colour(ap, w, vis0, vis1);
-        } else if constexpr (!kHash) {
-          const uint32_t id = __float_as_uint(srec[6][j].w);
-          const float* col = p.colors + (size_t)id * p.C;
-#pragma unroll
-          for (int c = 0; c < NACC; c++)
-            if (c < p.C) acc[c] = fmaf(col[c], w, acc[c]);
-        } else {
-          float xyz[3];
-          hit_world(srec[4][j], srec[5][j], srec[6][j], hit, xyz);
-          pos_x += w * xyz[0];
-          pos_y += w * xyz[1];
-          pos_z += w * xyz[2];
-          const uint32_t ap = __float_as_uint(q3.w);
-          float u[3];
-          bool oob;
-          grid_coord(g, xyz, u, oob);
-          const int slot = (qhead + qn) & (kQueue - 1);
-          hq[slot][threadIdx.x] = make_float4(u[0], u[1], u[2], w);
-          hl[slot][threadIdx.x] = hit_levels(oob, ap, L);
-          qn++;
-          float apc0, apc1;
-          if (ap <= 4u) {
-            apc0 = (float)((double)(uint32_t)(ap - 2u) * 0.5);
-            apc1 = 1.0f;
-          } else {
-            apc0 = 1.0f;
-            apc1 = (float)(1.0 - (double)(uint32_t)(ap - 4u) * 0.5);
-          }
-          vis0 += apc0 * w;
-          vis1 += apc1 * w;
-        }
-        T = test_T;
-        last_contributor = contributor;
-      } while (false);
+        const uint32_t j = j0 + (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1ull;
+        if (!done && splat_near(srec[0][j], srec[1][j], srec[2][j], srec[6][j].y, pxf, pyf))
+          hlist[cnt++][threadIdx.x] = (uint8_t)j;
+        if (__ballot(cnt == (uint32_t)kList)) break;
       }
-      if constexpr (kMix) {
-        // Render modes 4 and 13: the splat's feature row is read once per wave
-        // with one coalesced load (lane k holds entry k), then broadcast lane by
-        // lane; a lane's grid lookups go to its queue.
-        if (__ballot(ph.on) != 0ull) {
-          const uint32_t id = __builtin_amdgcn_readfirstlane(__float_as_uint(srec[6][j].w));
-          const float* row = p.colors + (size_t)id * (uint32_t)p.cstride;
-          const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
-          float mine = lane < (uint32_t)p.nrow ? row[lane] : 0.0f;
-          asm volatile("" : "+v"(mine));  // loaded here, with every lane active
-          const float wt = p.wslot >= 0 ? row[p.wslot] : 1.0f;
-          // fast hits skip the grid: weight > 0.5 in mode 13 inference, >= 0.9 in
-          // mode 12 inference (they take the row), < 0.1 in mode 14 inference and
-          // <= 1e-6 in mode 14 training (their grid levels stay zero)
-          const bool fast = (wt > p.fthr) != (p.fneg != 0);
-          if (ph.on) {
-            // per-splat channels at once; a fast hit's grid-level channels too
-            // when no earlier hit of the pixel is pending
-            const bool enq = !(fast && qn == 0);
-            const int ndirect = enq ? p.pgd : p.pgd + (int)p.nfast * F;
-#pragma unroll
-            for (int c = 0; c < NACC; c++) {
-              if (c < ndirect) {
-                const float rv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), c));
-                acc[c] = fmaf(p.wcoarse ? rv * wt : rv, ph.w, acc[c]);
-              }
+      for (;;) {
+        if (pos < cnt) {
+          const uint32_t j = hlist[pos++][threadIdx.x];
+          SplatHit hit;
+          do {
+            const float4 q6 = srec[6][j];
+            if (!splat_hit(srec[0][j], srec[1][j], srec[2][j], pxf, pyf, p.beta, hit, kKT ? p.kernel_type : 0, q6.z)) break;
+            const float test_T = T * (1 - hit.alpha);
+            if (test_T < 0.0001f) {
+              done = true;
+              pos = cnt;
+              break;
             }
-            const uint32_t ap = __float_as_uint(srec[3][j].w);
-            float u[3] = {0.0f, 0.0f, 0.0f};
-            uint32_t nh = 0u;
-            if (!fast || !p.m13) {  // a mode-13 fast hit has no world point
+            const float w = hit.alpha * T;
+            const uint32_t contributor = base + j + 1u;
+            render_number++;
+            if (p.max_intersections > 0 && render_number >= p.max_intersections) {
+              done = true;
+              pos = cnt;
+            }
+            const float4 q3 = srec[3][j];
+            const float depth = hit.depth;
+            const float Aa = 1 - T;
+            const float m = mfac * (1 - 0.2f / depth);
+            distortion += (m * m * Aa + M2 - 2 * m * M1) * w;
+            D += depth * w;
+            M1 += m * w;
+            M2 += m * m * w;
+            if (T > 0.5f) {
+              median_depth = depth;
+              median_contributor = (float)contributor;
+            }
+            N0 += q3.x * w;
+            N1 += q3.y * w;
+            N2 += q3.z * w;
+            T = test_T;
+            const uint32_t ap = __float_as_uint(q3.w);
+            const uint32_t id = __float_as_uint(q6.w);
+            if constexpr (kMix != 0) {
+              // Render modes 4, 12, 13 and 14: the leading channels from the
+              // splat's row, the grid's through the queue.
+              const float* row = p.colors + (size_t)id * (uint32_t)p.cstride;
+              const float wt = p.wslot >= 0 ? row[p.wslot] : 1.0f;
+              // fast hits skip the grid: weight > 0.5 in mode 13 inference, >= 0.9 in
+              // mode 12 inference (they take the row), < 0.1 in mode 14 inference and
+              // <= 1e-6 in mode 14 training (their grid levels stay zero)
+              const bool fast = (wt > p.fthr) != (p.fneg != 0);
+              // per-splat channels at once; a fast hit's grid-level channels too
+              // when no earlier hit of the pixel is pending
+              const bool enq = !(fast && qn == 0);
+              const int ndirect = enq ? p.pgd : p.pgd + (int)p.nfast * F;
+              row_accumulate<NACC>(p, row, ndirect, wt, w, acc);
+              float u[3] = {0.0f, 0.0f, 0.0f};
+              uint32_t nh = 0u;
+              if (!fast || !p.m13) {  // a mode-13 fast hit has no world point
+                float xyz[3];
+                hit_world(srec[4][j], srec[5][j], q6, hit, xyz);
+                pos_x += w * xyz[0];
+                pos_y += w * xyz[1];
+                pos_z += w * xyz[2];
+                if (!fast) {
+                  bool oob;
+                  grid_coord(g, xyz, u, oob);
+                  nh = hit_levels(oob, ap, L);
+                }
+              }
+              if (enq) {
+                const int slot = (qhead + qn) & (kQueue - 1);
+                hq[slot][threadIdx.x] = make_float4(u[0], u[1], u[2], w);
+                hm[slot][threadIdx.x] = id << 7 | (fast ? 64u : 0u) | nh;
+                qn++;
+              }
+              if (!p.m13) {
+                appearance_colour(ap, w, vis0, vis1);
+                // render mode 13 leaves the hit loop before the last-contributor update (CR/forward.cu:1097-1100)
+                last_contributor = contributor;
+              }
+            } else if constexpr (kHsh != 0) {
               float xyz[3];
-              hit_world(srec[4][j], srec[5][j], srec[6][j], ph.hit, xyz);
-              pos_x += ph.w * xyz[0];
-              pos_y += ph.w * xyz[1];
-              pos_z += ph.w * xyz[2];
-              if (!fast) {
-                bool oob;
-                grid_coord(g, xyz, u, oob);
-                nh = hit_levels(oob, ap, L);
+              hit_world(srec[4][j], srec[5][j], q6, hit, xyz);
+              pos_x += w * xyz[0];
+              pos_y += w * xyz[1];
+              pos_z += w * xyz[2];
+              const float* row = p.colors + (size_t)id * (uint32_t)p.cstride;
+              if constexpr (kHsh == 1 || kHsh == 5) {
+                surface_accumulate<kHsh, NACC>(p, xyz, ap, q3, row, w, acc);
+              } else {
+                float h[3];
+                if (p.hsh_dec != 1)
+                  hsh_query(g, xyz, ap, h);
+                else
+                  h[0] = h[1] = h[2] = 0.0f;
+                hsh_accumulate<kHsh, NACC>(p, row, h, w, acc);
               }
-            }
-            if (enq) {
+              appearance_colour(ap, w, vis0, vis1);
+              last_contributor = contributor;
+            } else if constexpr (!kHash) {
+              const float* col = p.colors + (size_t)id * p.C;
+#pragma unroll
+              for (int c = 0; c < NACC; c++)
+                if (c < p.C) acc[c] = fmaf(col[c], w, acc[c]);
+              last_contributor = contributor;
+            } else {
+              float xyz[3];
+              hit_world(srec[4][j], srec[5][j], q6, hit, xyz);
+              pos_x += w * xyz[0];
+              pos_y += w * xyz[1];
+              pos_z += w * xyz[2];
+              float u[3];
+              bool oob;
+              grid_coord(g, xyz, u, oob);
               const int slot = (qhead + qn) & (kQueue - 1);
-              hq[slot][threadIdx.x] = make_float4(u[0], u[1], u[2], ph.w);
-              hm[slot][threadIdx.x] = id << 7 | (fast ? 64u : 0u) | nh;
+              hq[slot][threadIdx.x] = make_float4(u[0], u[1], u[2], w);
+              const uint32_t nlev = hit_levels(oob, ap, L);
+              // the part's share of the levels below nlev (parts is a power of two)
+              hl[slot][threadIdx.x] =
+                  (uint8_t)(!kParts || p.parts == 1u ? nlev
+                                                     : nlev > part ? (nlev - part + p.parts - 1u) >> p.parts_log2 : 0u);
               qn++;
+              appearance_colour(ap, w, vis0, vis1);
+              last_contributor = contributor;
             }
-            if (!p.m13) appearance_colour(ap, ph.w, vis0, vis1);
-            T = ph.T;
-            // render mode 13 leaves the hit loop before the last-contributor update (CR/forward.cu:1097-1100)
-            if (!p.m13) last_contributor = contributor;
+          } while (false);
+        }
+        if constexpr (kHash) {
+          // whenever a lane is full; at the end, until every queue is empty
+          if (__ballot(qn == kQueue) || (last && __ballot(qn > 0))) {
+            if constexpr (kMix && F <= 4)
+              drain_compact_mix<F, NACC, kHalf, kStructured, kMix == 2>(p, rsrc, hq, hm, isrc + wid * kWaveLanes,
+                                                                        qhead, qn, acc);
+            else if constexpr (kMix)
+              drain_mixed<F, NACC, kHalf, kStructured, kMix == 2>(p, rsrc, hq, hm, qhead, qn, acc);
+            else if constexpr (F <= 4)
+              drain_compact<F, NACC, kHalf, kStructured>(g, part, kParts ? p.parts : 1u, rsrc, hq, hl,
+                                                         isrc + wid * kWaveLanes, qhead, qn, acc);
+            else
+              drain_round<F, NACC, kHalf, kStructured>(g, rsrc, hq, hl, qhead, qn, acc);
+            if (last) continue;
           }
         }
+        if (__ballot(pos < cnt) == 0ull) break;
       }
-      j++;
-      if (kHash && __ballot(qn == kQueue)) break;
-      if (__ballot(!done) == 0) j = n;
-    }
-    const bool batch_end = j >= n;
-    if constexpr (kHash) {
-      // whenever a lane is full; at the end, until every queue is empty
-      if (__ballot(qn == kQueue) || (last && __ballot(qn > 0))) {
-        if constexpr (kMix && F <= 4)
-          drain_compact_mix<F, NACC, kHalf, kStructured, kMix == 2>(p, rsrc, hq, hm, isrc + wid * kWaveLanes, qhead,
-                                                                    qn, acc);
-        else if constexpr (kMix)
-          drain_mixed<F, NACC, kHalf, kStructured, kMix == 2>(p, rsrc, hq, hm, qhead, qn, acc);
-        else if constexpr (F <= 4)
-          drain_compact<F, NACC, kHalf, kStructured>(g, rsrc, hq, hl, isrc + wid * kWaveLanes, qhead, qn, acc);
-        else
-          drain_round<F, NACC, kHalf, kStructured>(g, rsrc, hq, hl, qhead, qn, acc);
-        if (last) continue;
-      }
-    }
-    if (batch_end) break;
+      if (last || (todo == 0ull && chunk == (uint32_t)kWaves) || __ballot(!done) == 0ull) break;
     }
     if (last) break;
     start += kBatch;
@@ -957,21 +1021,34 @@ render_kernel(const RenderParams p) {
   if (!inside) return;
   const size_t HW = (size_t)p.W * p.H;
   const size_t pid = (size_t)p.W * py + px;
+  if constexpr (kParts) {
+    if (p.parts > 1u) {
+#pragma unroll
+      for (int c = 0; c < NACC; c++) {
+        const int oc = (int)(part + (uint32_t)(c / F) * p.parts) * F + c % F;
+        if (oc < p.C) p.out_color[(size_t)oc * HW + pid] = acc[c];
+      }
+      if (part != 0u) return;
+      for (int c = (int)(p.parts * p.part_levels) * F; c < p.C; c++) p.out_color[(size_t)c * HW + pid] = 0.0f;
+    }
+  }
   p.final_T[pid] = T;
   p.final_T[pid + HW] = M1;
   p.final_T[pid + 2 * HW] = M2;
   p.n_contrib[pid] = last_contributor;
   p.n_contrib[pid + HW] = f2u_sat(median_contributor);
+  const bool whole = !kParts || p.parts == 1u;
 #pragma unroll
   for (int c = 0; c < NACC; c++) {
-    if (c < p.C) {
+    if (whole && c < p.C) {
       int oc = c;
       if constexpr (kMix != 0)
         if (c < p.rot_n) oc = (c + p.rot) % p.rot_n;  // render mode 2: the grid's channels first
       p.out_color[(size_t)oc * HW + pid] = acc[c];
     }
   }
-  for (int c = NACC; c < p.C; c++) p.out_color[(size_t)c * HW + pid] = 0.0f;
+  if (whole)
+    for (int c = NACC; c < p.C; c++) p.out_color[(size_t)c * HW + pid] = 0.0f;
   float* O = p.out_others;
   O[pid + 0 * HW] = D;
   O[pid + 1 * HW] = 1 - T;
@@ -1039,9 +1116,8 @@ __global__ void __launch_bounds__(kRenderThreads) record_transmittance_kernel(co
           const float4 bb = sgeo[3][j];
           if (bb.y < wx0 || bb.x > wx1 || bb.w < wy0 || bb.z > wy1) break;
           SplatHit hit;
-          if (!splat_hit(sgeo[0][j], sgeo[1][j], sgeo[2][j], sgeo[4][j].y, pxf, pyf, p.beta, hit, p.kernel_type,
-                         sgeo[4][j].z))
-            break;
+          if (!splat_near(sgeo[0][j], sgeo[1][j], sgeo[2][j], sgeo[4][j].y, pxf, pyf)) break;
+          if (!splat_hit(sgeo[0][j], sgeo[1][j], sgeo[2][j], pxf, pyf, p.beta, hit, p.kernel_type, sgeo[4][j].z)) break;
           const float test_T = T * (1 - hit.alpha);
           if (test_T < 0.0001f) {
             done = true;
@@ -1201,14 +1277,21 @@ hipError_t launch_spatial_add(const RenderParams& p, const float* ap_level, hipS
 template <int F, int NACC, bool kHash, bool kHalf, bool kStructured = false, int kMix = 0, bool kKT = false,
           int kHsh = 0>
 static hipError_t launch_one(const RenderParams& p, hipStream_t s) {
-  hipLaunchKernelGGL((render_kernel<F, NACC, kHash, kHalf, kStructured, kMix, kKT, kHsh>), dim3(p.ntiles),
+  const uint32_t blocks = p.parts > 1u ? (p.ntiles + 7u) / 8u * 8u * p.parts : p.ntiles;
+  hipLaunchKernelGGL((render_kernel<F, NACC, kHash, kHalf, kStructured, kMix, kKT, kHsh>), dim3(blocks),
                      dim3(kRenderThreads), 0, s, p);
   return hipGetLastError();
 }
 
 template <int F, bool kHalf, bool kStructured, bool kKT>
 static hipError_t launch_hash_levels(const RenderParams& p, hipStream_t s) {
-  const uint32_t L = p.grid.L;
+  const uint32_t L = p.part_levels;
+  if constexpr (kStructured && !kKT && F <= 4) {
+    if (p.parts > 1u) {
+      if (L <= 2) return launch_one<F, F * 2, true, kHalf, kStructured, 0, kKT>(p, s);
+      if (L <= 4) return launch_one<F, F * 4, true, kHalf, kStructured, 0, kKT>(p, s);
+    }
+  }
   if constexpr (F * 8 <= NEST_MAX_CHANNELS)
     if (L <= 8) return launch_one<F, F * 8, true, kHalf, kStructured, 0, kKT>(p, s);
   if constexpr (F * 16 <= NEST_MAX_CHANNELS)
@@ -1241,8 +1324,21 @@ __device__ __forceinline__ uint32_t order_bin(uint32_t n) {
 
 constexpr int kOrderHeld = 16;  // tiles per thread whose bins stay in registers (16384 tiles)
 
+// The level records of a structured grid ride along in the kernel arguments
+// and are copied to device memory, where the render reads them with scalar
+// loads.
+struct LevelQuads {
+  LevelQuad q[NEST_MAX_LEVELS];
+};
+
 __global__ void __launch_bounds__(kOrderThreads) tile_order_kernel(const uint2* ranges, uint32_t ntiles,
-                                                                  uint32_t* order) {
+                                                                  uint32_t* order, LevelQuads lq, uint32_t L,
+                                                                  LevelQuad* lq_dst) {
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int l = 0; l < NEST_MAX_LEVELS; l++)
+      if ((uint32_t)l < L) lq_dst[l] = lq.q[l];
+  }
   static_assert(kOrderBins == 4 * kWaveLanes, "four bins per lane in the scan");
   __shared__ uint32_t cnt[kOrderBins];
   for (int b = threadIdx.x; b < kOrderBins; b += kOrderThreads) cnt[b] = 0u;
@@ -1311,19 +1407,6 @@ __global__ void __launch_bounds__(kOrderThreads) tile_order_kernel(const uint2* 
   }
 }
 
-struct LevelQuads {
-  LevelQuad q[NEST_MAX_LEVELS];
-};
-
-// Copies the level records from the kernel arguments to device memory, where
-// the render reads them with scalar loads.
-__global__ void level_quads_kernel(LevelQuads lq, uint32_t L, LevelQuad* dst) {
-  if (threadIdx.x != 0) return;
-#pragma unroll
-  for (int l = 0; l < NEST_MAX_LEVELS; l++)
-    if ((uint32_t)l < L) dst[l] = lq.q[l];
-}
-
 // Accumulators of the per-splat feature modes: the output levels the mode
 // writes (hyb + L, or the row's levels in mode 13), 32 or 64 channels.
 template <int F, bool kHalf, bool kStructured, bool kKT>
@@ -1350,19 +1433,6 @@ static hipError_t launch_hash(const RenderParams& p, hipStream_t s) {
     return launch_hash_levels<F, kHalf, false, kKT>(p, s);
   }
   if constexpr (!kKT) {
-    const GridParams& g = p.grid;
-    LevelQuads lq = {};
-    for (uint32_t l = 0; l < g.L; l++) {
-      LevelQuad& q = lq.q[l];
-      q.scale = g.lv.scale[l];
-      const bool dense = l < g.n_dense;
-      q.a = dense ? g.lv.res1[l] : g.lv.hsize[l] - 1u;
-      q.b = dense ? g.lv.res1[l] * g.lv.res1[l] : 0u;
-      q.soff = g.lv.base[l] * (uint32_t)(F * (kHalf ? 2 : 4));
-    }
-    hipLaunchKernelGGL(level_quads_kernel, dim3(1), dim3(64), 0, s, lq, g.L, g.lq);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
     if constexpr (F >= 2) {
       if (p.mix) return launch_mix_levels<F, kHalf, true, false>(p, s);
     }
@@ -1405,9 +1475,47 @@ hipError_t launch_render(const RenderParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-static hipError_t launch_render_kernel(const RenderParams& p, hipStream_t s) {
+// Workgroups per tile, each with every parts-th level of the grid.  A tile's
+// walk and its lookups are one chain per pixel, so a frame of few tiles leaves
+// the chip idle, and a frame of up to ~2500 tiles ends on a thin last round;
+// parts repeat the compositing (0.4 of the 2.8 ms of the 100k-splat 800 x 800
+// frame) and split the lookups, each XCD keeping to one part's tables.  The
+// levels are dealt round-robin because the fine ones cost most (contiguous
+// halves: 3.70 ms where the dealt ones take 2.33).  Measured, render ms with
+// 1 / 2 / 4 / 8 parts, 16 levels: 64 tiles 0.94 / 0.69 / 0.57 / 0.49; 256
+// tiles 1.11 / 0.79 / 0.70 / 0.95; 625 tiles 1.32 / 1.02 / 1.25 / 1.91 and 1.66
+// / 1.48 / 1.55 / 2.17; 1200 tiles 2.03 / 1.80 / 2.19; 2500 tiles 2.91 / 2.33 /
+// 2.71 (object), 2.28 / 2.35 / 3.06 and 2.99 / 2.72 / 3.42 (unbounded); 4056
+// tiles 3.60 / 3.90 / 5.34.  8 levels: 64 tiles 0.68 / 0.55 / 0.48 / 0.47; 256
+// tiles 0.70 / 0.58 / 0.55 / 0.88; 625 tiles 0.71 / 0.63 / 0.99; 1200 tiles
+// 0.94 / 1.08 / 1.61.
+static uint32_t level_parts(uint32_t tiles, uint32_t L) {
+  if (L > 8u) return tiles <= 96u ? 8u : tiles <= 400u ? 4u : tiles <= 2560u ? 2u : 1u;
+  if (L >= 4u) return tiles <= 320u ? 4u : tiles <= 768u ? 2u : 1u;
+  return 1u;
+}
+
+static hipError_t launch_render_kernel(const RenderParams& p0, hipStream_t s) {
+  RenderParams p = p0;
+  const GridParams& g = p.grid;
+  const bool plain = p.level != 0 && !p.mix && p.hsh == 0;
+  const bool quads = g.structured && p.kernel_type == 0 && (plain || p.mix);
+  p.parts = plain && quads && g.F <= 4u ? level_parts(p.ntiles, g.L) : 1u;
+  p.part_levels = (g.L + p.parts - 1u) / p.parts;
+  p.parts_log2 = (uint32_t)__builtin_ctz(p.parts);
+  LevelQuads lq = {};
+  if (quads) {
+    for (uint32_t l = 0; l < g.L; l++) {
+      LevelQuad& q = lq.q[l];
+      q.scale = g.lv.scale[l];
+      const bool dense = l < g.n_dense;
+      q.a = dense ? g.lv.res1[l] : g.lv.hsize[l] - 1u;
+      q.b = dense ? g.lv.res1[l] * g.lv.res1[l] : 0u;
+      q.soff = g.lv.base[l] * (g.F * (g.half ? 2u : 4u));
+    }
+  }
   hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(kOrderThreads), 0, s, reinterpret_cast<const uint2*>(p.ranges),
-                     p.ntiles, p.tile_order);
+                     p.ntiles, p.tile_order, lq, quads ? g.L : 0u, g.lq);
   const hipError_t oe = hipGetLastError();
   if (oe != hipSuccess) return oe;
   if (p.mix && p.grid.F == 1) return hipErrorInvalidValue;

@@ -321,3 +321,26 @@ def test_kernel_types_parity(oracle, name, kt):
     check_record(res, r)
     gauss = run_gpu(sc)
     assert not np.array_equal(gauss.others.cpu().numpy()[7], r["others"][7])  # the kernel changed the hits
+
+
+# (W, H, L, F, half table): tile counts on both sides of each line of the
+# level-parts rule (96, 400 and 2560 tiles over 8 levels, 320 and 768 up to
+# 8), level counts that the parts do not divide, and 2 levels (no parts)
+PART_CASES = [(96 * 16, 16, 16, 2, False), (97 * 16 - 3, 13, 11, 4, False), (20 * 16, 20 * 16, 9, 4, True),
+              (401 * 16 - 15, 9, 16, 2, False), (64 * 16, 40 * 16, 13, 1, False), (197 * 16, 13 * 16 - 7, 16, 2, False),
+              (320 * 16, 16, 8, 2, False), (321 * 16, 15, 5, 4, False), (96 * 16, 8 * 16, 7, 2, True),
+              (769 * 16, 10, 8, 4, True), (40, 24, 4, 2, False), (40, 24, 2, 4, False), (1, 1, 16, 4, False)]
+
+
+@pytest.mark.parametrize("W,H,L,F,half", PART_CASES)
+def test_level_parts_parity(oracle, W, H, L, F, half):
+    from nest_splat.scene import get_spec, make_scene
+    print(f"[case] parts {W}x{H} L={L} F={F} half={half}", flush=True)
+    sc = make_scene(get_spec("cfg2", name="parts", P=6000, W=W, H=H, L=L, F=F, log2T=12, log_scale_mu=-3.0,
+                             table_dtype="f16" if half else "f32"))
+    _, _, r = run_oracle(oracle, sc)
+    res = run_gpu(sc)
+    np.testing.assert_array_equal(res.color.cpu().numpy(), r["color"])
+    np.testing.assert_array_equal(res.others.cpu().numpy(), r["others"])
+    if W * H > 1000:
+        assert r["others"][7].sum() > 100
