@@ -11,13 +11,15 @@
 //
 // Layout of the render backward: one 256-thread workgroup per 16x16 tile, one
 // lane per pixel, the tile's splats walked back to front in LDS-staged
-// batches of the forward's packed records.  With a grid, a wave splits each
-// batch into segments: a geometry pass queues the segment's hits, the queued
+// batches of the forward's packed records, of which a wave looks at those
+// whose acceptance bbox meets its 16 x 4 pixels (masks balloted while staging)
+// and that precede a pixel's last contributor.  With a grid, a wave splits
+// each batch into segments: a hit pass queues the segment's hits, the queued
 // hits are spread one per lane for the grid work (table gathers, the
 // features' dot product with dL/dpixel, dL/dxyz, the table-gradient scatter),
-// and a third pass runs the blending recursion over the splats that hit the
-// wave.  Two restructurings against the reference, both the same sums in
-// another order:
+// and a third pass runs the blending recursion, each lane over its own hits.
+// Two restructurings against the reference, both the same sums in another
+// order:
 //  - the reference keeps three C-long arrays per pixel (accum_rec,
 //    last_color, dL_dpixel).  The back-to-front blend accum_rec =
 //    a*last + (1-a)*accum_rec is linear with the same coefficients for every
@@ -26,10 +28,10 @@
 //    products with dL_dpixel) and reads its dL_dpixel values from memory
 //    where a level needs them (cache-resident, coalesced across the wave);
 //    the |grad| sum of a hit is w * sum |dL_dpixel|, summed once per pixel;
-//  - every lane of a wave visits the same staged splat at the same time, so
-//    the per-splat gradients (transmat, homotrans, mean2D, normal, opacity,
-//    |grad| sum, colours) are summed over the wave with cross-lane shuffles
-//    and added with one atomic per wave instead of one per pixel.
+//  - the per-splat gradients (transmat, homotrans, mean2D, normal, opacity,
+//    |grad| sum, colours) are summed per staged batch in LDS over the tile's
+//    256 pixels and added to memory once, a splat's consecutive values by
+//    consecutive lanes, instead of one atomic per pixel and value.
 // Table gradients are hardware float atomics (global_atomic_add_f32) at
 // every corner, as in the reference, merged per cell across the wave first.
 // Their cost is one request per (instruction, 64-byte segment) and, on
@@ -41,6 +43,7 @@
 #include "hashgrid.h"
 #include "nest_internal.h"
 #include "nest_math.h"
+#include "splat_near.h"
 
 namespace nest {
 
@@ -257,11 +260,11 @@ template <int F>
 __device__ __forceinline__ void hash_backward_wave(const GridParams& g, nest_i32x4 rsrc, const float u[3],
                                                    float grad_scale, uint32_t lane_levels, float w,
                                                    const float* dpix, size_t HW, float* dtable, uint32_t* st,
-                                                   float& dot, float dxyz[3]) {
+                                                   uint32_t first, uint32_t step, float& dot, float dxyz[3]) {
   dot = 0.0f;
   dxyz[0] = dxyz[1] = dxyz[2] = 0.0f;
   const LevelTable& lv = g.lv;
-  for (int l = 0; l < (int)g.L; l++) {
+  for (int l = (int)first; l < (int)g.L; l += (int)step) {
     const bool on = (uint32_t)l < lane_levels;
     if (__ballot(on) == 0ull) break;  // levels are a prefix per lane
     const float scale = lv.scale[l];
@@ -640,13 +643,273 @@ __device__ __forceinline__ void bwd_hit_grad(BwdPixel& px, const BwdHit& h, cons
   gr.gO = h.G * dL_dalpha;
 }
 
-// The wave's per-splat sums (every lane takes part; lanes without a hit add
-// zeros) and one atomic per wave, splat and value.  gS is the |grad| sum,
-// wcol the colour weight (colour path and the per-splat rows), wt the row's
-// blend weight and fdot dL/dweight (render modes 7, 12 and 14).
-template <bool kHash, int kRows>
-__device__ __forceinline__ void bwd_splat_sums(const RenderBwdParams& p, const BwdPixel& px, uint32_t id, bool act,
-                                               const BwdGrad& gr, float gS, float wcol, float wt, float fdot) {
+// Per-splat gradient sums of a staged batch, kept in LDS over the tile's four
+// waves and added to memory once per batch: one row of values per splat, rows
+// of an odd length so that the lanes' splats spread over the banks.
+constexpr uint32_t kSumT = 0, kSumM = 9, kSumN = 11, kSumO = 14, kSumK = 15;
+constexpr uint32_t kSumCol = 16, kSumColour = 19;             // colour path: 3 colours
+constexpr uint32_t kSumH = 16, kSumS = 25, kSumW = 26, kSumHash = 27;  // grid path
+
+__device__ __forceinline__ void lds_add(float* a, float v) {
+  __hip_atomic_fetch_add(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+constexpr uint32_t kBigGroup = 8;   // lanes at one splat that are summed in registers first
+
+// Rest of a reduce-scatter of 32 values over the wave after its first step
+// (values i and i + 16 halved over lane bit 5 into r[i]): r[0] is then the sum
+// over the lanes of value l / 2, whose index is returned.
+__device__ __forceinline__ uint32_t reduce_scatter16(float (&r)[16]) {
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t vi = (lane >> 5) * 16u;
+#pragma unroll
+  for (int s = 1; s < 5; s++) {
+    const int h = 16 >> s;
+#pragma unroll
+    for (int i = 0; i < h; i++) r[i] = halve(5 - s, r[i], r[i + h]);
+    if (((lane >> (5 - s)) & 1u) != 0u) vi += (uint32_t)h;
+  }
+  r[0] = halve(0, r[0], r[0]);
+  return vi;
+}
+
+// Adds the lanes' N values (those with `on`) to the sums of their splats j.
+// Lanes at the same splat are common where splats are wide (every lane of a
+// wave walks the same depth order), and LDS adds to one address run one after
+// the other, so a splat with kBigGroup lanes or more is summed over them with
+// a recursive-halving reduce-scatter (after it lane l holds value l / 2) and
+// added by one instruction; the other lanes add for themselves.  (Groups from
+// 4 / 8 / 16 lanes: 1.13 / 1.10 / 1.31 ms on the colour path's frame.)
+template <uint32_t N>
+__device__ __forceinline__ void bwd_add_row(bool on, uint32_t j, const float (&v)[N], float* sums) {
+  static_assert(N > 16 && N <= 32, "one reduce-scatter of 32 values");
+  const uint32_t lane = threadIdx.x & 63u;
+  uint64_t rem = __ballot(on);
+  bool single = on;
+  while (rem != 0ull) {
+    const int ld = __ffsll((long long)rem) - 1;
+    const uint32_t jl = (uint32_t)__builtin_amdgcn_readlane((int)j, ld);
+    const uint64_t m = __ballot(j == jl) & rem;
+    rem &= ~m;
+    if ((uint32_t)__popcll(m) < kBigGroup) continue;
+    const bool mem = ((m >> lane) & 1ull) != 0ull;
+    single = single && !mem;
+    float r[16];
+#pragma unroll
+    for (uint32_t i = 0; i < 16; i++) r[i] = halve(5, mem ? v[i] : 0.0f, i + 16 < N ? (mem ? v[i + 16] : 0.0f) : 0.0f);
+    const uint32_t vi = reduce_scatter16(r);
+    if ((lane & 1u) == 0u && vi < N) lds_add(sums + jl * N + vi, r[0]);
+  }
+  if (single) {
+#pragma unroll
+    for (uint32_t i = 0; i < N; i++)
+      if (v[i] != 0.0f) lds_add(sums + j * N + i, v[i]);
+  }
+}
+
+// The values every path sends to a splat.
+__device__ __forceinline__ void bwd_row_geometry(const BwdGrad& gr, float* v) {
+#pragma unroll
+  for (uint32_t r = 0; r < 9; r++) v[kSumT + r] = gr.gT[r];
+  v[kSumM] = gr.gM[0];
+  v[kSumM + 1] = gr.gM[1];
+#pragma unroll
+  for (uint32_t r = 0; r < 3; r++) v[kSumN + r] = gr.gN[r];
+  v[kSumO] = gr.gO;
+  v[kSumK] = gr.gK;
+}
+
+// Adds n consecutive sums of every staged splat to dst rows of `stride`
+// floats and clears them; consecutive lanes take consecutive floats of a row.
+template <uint32_t kRow, uint32_t n>
+__device__ __forceinline__ void bwd_flush(float* sums, uint32_t first, uint32_t splats, const uint32_t* sid, float* dst,
+                                          uint32_t stride) {
+  for (uint32_t i = threadIdx.x; i < splats * n; i += kBwdThreads) {
+    const uint32_t j = i / n, r = i % n;
+    float* a = sums + j * kRow + first + r;
+    const float v = *a;
+    if (v != 0.0f) {
+      *a = 0.0f;
+      atomic_add(dst + (size_t)sid[j] * stride + r, v);
+    }
+  }
+}
+
+template <uint32_t kRow>
+__device__ __forceinline__ void bwd_flush_geometry(const RenderBwdParams& p, float* sums, uint32_t splats,
+                                                   const uint32_t* sid) {
+  bwd_flush<kRow, 9>(sums, kSumT, splats, sid, p.dtransmat, 9);
+  bwd_flush<kRow, 2>(sums, kSumM, splats, sid, p.dmean2D, 3);
+  bwd_flush<kRow, 3>(sums, kSumN, splats, sid, p.dnormal, 3);
+  bwd_flush<kRow, 1>(sums, kSumO, splats, sid, p.dopacity, 1);
+  if (p.dshapes != nullptr) bwd_flush<kRow, 1>(sums, kSumK, splats, sid, p.dshapes, 1);
+}
+
+constexpr int kBwdCand = 8;  // candidate splats a pixel holds between the test and the hit pass
+constexpr int kBwdWaves = kBwdThreads / 64;
+
+// Masks of the staged splats whose acceptance bbox meets each wave's 16 x 4
+// pixel block; one call per 64 splats, by the wave that staged them.
+template <int kChunks>
+__device__ __forceinline__ void bwd_block_masks(bool in, const float4& bb, uint32_t tx, uint32_t ty, uint32_t chunk,
+                                                uint64_t (*smask)[kChunks]) {
+  const float bx0 = (float)(tx * kTile), bx1 = bx0 + 15.0f;
+#pragma unroll
+  for (int b = 0; b < kBwdWaves; b++) {
+    const float by0 = (float)(ty * kTile + 4 * b), by1 = by0 + 3.0f;
+    const uint64_t m = __ballot(in && !(bb.y < bx0 || bb.x > bx1 || bb.w < by0 || bb.z > by1));
+    if ((threadIdx.x & 63u) == 0u) smask[b][chunk] = m;
+  }
+}
+
+__device__ __forceinline__ uint64_t wave_u64(uint64_t m) {
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)m) |
+         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(m >> 32)) << 32;
+}
+
+// Largest of the lanes' values, in every lane.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, 64));
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+
+constexpr uint32_t kWideSplat = 24;  // candidate lanes from which a splat is taken by the whole wave
+
+// Colour path with 3 channels (SH colours, RGB).  A wave lists each pixel's
+// candidates (splats whose bbox meets its block, in front of the pixel's last
+// contributor, conservative test), back to front, then every lane works
+// through its own list: exact test, blending recursion, gradients into the
+// batch's LDS sums.  A splat of kWideSplat candidates or more is taken by all
+// of them at once (lists let the lanes drift apart, which splits its sum).  Bound by the recursion's serial arithmetic and the ~15
+// LDS adds per hit.  The lockstep walk below visits every splat of the tile
+// with 18 wave sums and atomics per splat; 200k splats, SH degree 3, 800x800:
+// 2.92 ms there, 1.17 ms here (2.26 with every lane adding for itself: LDS adds
+// to one address run one after the other).
+__global__ void __launch_bounds__(kBwdThreads) render_backward_rgb_kernel(const RenderBwdParams p) {
+  __shared__ float4 srec[4][kBwdThreads];  // record chunks 0-3, the shape in place of the appearance level
+  __shared__ float scut[kBwdThreads];
+  __shared__ uint32_t sid[kBwdThreads];
+  __shared__ float sums[kBwdThreads * kSumColour];
+  __shared__ uint8_t hlist[kBwdCand][kBwdThreads];
+  __shared__ uint64_t smask[kBwdWaves][kBwdWaves];
+  __shared__ uint32_t slast[kBwdWaves];
+
+  const uint32_t tile = p.tile_order[blockIdx.x];  // the forward's order: heaviest tiles first
+  const uint2 range = reinterpret_cast<const uint2*>(p.ranges)[tile];
+  if (range.x >= range.y) return;
+  const size_t HW = (size_t)p.W * p.H;
+  const uint32_t tx = tile % p.gx, ty = tile / p.gx;
+  const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  BwdPixel px;
+  bwd_pixel_init(p, tile, px);
+  float dpix[3];
+#pragma unroll
+  for (int c = 0; c < 3; c++) dpix[c] = px.inside ? px.dpix[(size_t)c * HW] : 0.0f;
+  for (uint32_t i = threadIdx.x; i < kBwdThreads * kSumColour; i += kBwdThreads) sums[i] = 0.0f;
+  const uint32_t wlast = wave_max(px.last_contributor);
+  if ((threadIdx.x & 63u) == 0u) slast[wid] = wlast;
+  __syncthreads();
+  const uint32_t total = range.y - range.x;
+  const uint32_t tlast = min(total, max(max(slast[0], slast[1]), max(slast[2], slast[3])));
+  // batches of splats tlast .. 1 of the tile's list; index j is splat below - j
+  for (uint32_t below = tlast; below > 0u; below -= min(below, (uint32_t)kBwdThreads)) {
+    const uint32_t n = min((uint32_t)kBwdThreads, below);
+    const bool in = threadIdx.x < n;
+    float4 bb = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (in) {
+      const uint32_t id = p.point_list[range.x + below - 1u - threadIdx.x];
+      const float4* rec = reinterpret_cast<const float4*>(p.records) + 8 * (size_t)id;
+#pragma unroll
+      for (int c = 0; c < 3; c++) srec[c][threadIdx.x] = rec[c];
+      const float4 q6 = rec[6];
+      float4 q3 = rec[3];
+      q3.w = q6.z;
+      srec[3][threadIdx.x] = q3;
+      scut[threadIdx.x] = q6.y;
+      sid[threadIdx.x] = id;
+      bb = rec[7];
+    }
+    bwd_block_masks<kBwdWaves>(in, bb, tx, ty, wid, smask);
+    __syncthreads();
+    uint64_t todo = 0ull;  // splats of the current 64 still to be visited
+    uint32_t chunk = 0u, j0 = 0u;
+    uint32_t cnt = 0u, pos = 0u;  // the lane's listed splats, the next of them
+    bool flush = false;           // work through the lists
+    for (;;) {
+      bool on = false;
+      uint32_t j = 0u;
+      if (flush) {
+        on = pos < cnt;
+        if (__ballot(on) == 0ull) {
+          if (todo == 0ull && chunk == (uint32_t)kBwdWaves) break;
+          cnt = pos = 0u;
+          flush = false;
+          continue;
+        }
+        if (on) j = hlist[pos++][threadIdx.x];
+      } else {
+        if (todo == 0ull) {
+          flush = chunk == (uint32_t)kBwdWaves;
+          if (!flush) {
+            todo = wave_u64(smask[wid][chunk]);
+            j0 = chunk++ * 64u;
+          }
+          continue;
+        }
+        j = j0 + (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1ull;
+        // the splat is number below - j of the tile's list, from 1
+        const bool near = below - j <= px.last_contributor &&
+                          splat_near(srec[0][j], srec[1][j], srec[2][j], scut[j], px.pxf, px.pyf);
+        const uint64_t m = __ballot(near);
+        if (m == 0ull) continue;
+        const bool wide = (uint32_t)__popcll(m) >= kWideSplat;
+        if (!wide || __ballot(cnt != 0u) != 0ull) {
+          if (near) hlist[cnt++][threadIdx.x] = (uint8_t)j;
+          flush = wide || __ballot(cnt == (uint32_t)kBwdCand) != 0ull;
+          continue;
+        }
+        on = near;  // a wide splat with no list pending: at once
+      }
+      bool hit = false;
+      float v[kSumColour];
+#pragma unroll
+      for (uint32_t i = 0; i < kSumColour; i++) v[i] = 0.0f;
+      if (on) {
+        const float4 q1 = srec[1][j], q2 = srec[2][j], q3 = srec[3][j];
+        BwdHit h;
+        hit = bwd_hit(srec[0][j], q1, q2, px.pxf, px.pyf, p.beta, true, h, p.kernel_type, q3.w);
+        if (hit) {
+          px.T = px.T / (1.f - h.alpha);
+          const float wgt = h.alpha * px.T;
+          const float* col = p.colors + 3 * (size_t)sid[j];
+          float dot = 0.0f;
+#pragma unroll
+          for (int c = 0; c < 3; c++) dot += col[c] * dpix[c];
+          BwdGrad gr;
+          bwd_grad_zero(gr);
+          const float dxyz[3] = {0.0f, 0.0f, 0.0f};
+          bwd_hit_grad<false>(px, h, q1, q2, q3, q3, q3, p.beta, below - j - 1u, dot, dxyz, gr, p.kernel_type);
+          bwd_row_geometry(gr, v);
+#pragma unroll
+          for (uint32_t c = 0; c < 3; c++) v[kSumCol + c] = wgt * dpix[c];
+        }
+      }
+      bwd_add_row<kSumColour>(hit, j, v, sums);
+    }
+    __syncthreads();
+    bwd_flush_geometry<kSumColour>(p, sums, n, sid);
+    bwd_flush<kSumColour, 3>(sums, kSumCol, n, sid, p.dcolors, 3);
+    __syncthreads();
+  }
+}
+
+// Colour path with any channel count: the wave walks the staged splats back
+// to front in lockstep, every lane one pixel, with the per-splat sums over the
+// wave and one atomic per wave, splat and value.
+__device__ __forceinline__ void bwd_splat_sums(const RenderBwdParams& p, const BwdPixel& px, uint32_t id,
+                                               const BwdGrad& gr, float wcol) {
   const size_t HW = (size_t)p.W * p.H;
   const float* dpix = px.dpix;
   const bool lead = (threadIdx.x & 63u) == 0u;
@@ -655,33 +918,9 @@ __device__ __forceinline__ void bwd_splat_sums(const RenderBwdParams& p, const B
     const float v = wave_sum(gr.gT[r]);
     if (lead && v != 0.0f) atomic_add(p.dtransmat + 9 * (size_t)id + r, v);
   }
-  if constexpr (kHash) {
-#pragma unroll
-    for (int r = 0; r < 9; r++) {
-      const float v = wave_sum(gr.gH[r]);
-      if (lead && v != 0.0f) atomic_add(p.dhomo + 9 * (size_t)id + r, v);
-    }
-    const float vs = wave_sum(gS);
-    if (lead && vs != 0.0f) atomic_add(p.gradsum + id, vs);
-    if constexpr (kRows == 1) {
-      for (int ch = 0; ch < p.pgd; ch++) {
-        const float v = wave_sum(wcol * dpix[(size_t)ch * HW]);
-        if (lead && v != 0.0f) atomic_add(p.dcolors + (size_t)id * p.pgd + ch, v);
-      }
-    } else if constexpr (kRows == 2) {
-      float* dc = p.dcolors + (size_t)id * (uint32_t)p.cstride;
-      for (int ch = 0; ch < p.pgd + (p.azero ? 0 : p.nfine); ch++) {
-        const float v = wave_sum((ch < p.pgd ? wcol : wcol * wt) * dpix[(size_t)ch * HW]);
-        if (lead && v != 0.0f) atomic_add(dc + ch, v);
-      }
-      const float vw = wave_sum(act ? fdot : 0.0f);
-      if (lead && vw != 0.0f) atomic_add(dc + p.wslot, vw);
-    }
-  } else {
-    for (int ch = 0; ch < p.C; ch++) {
-      const float v = wave_sum(px.inside ? wcol * dpix[(size_t)ch * HW] : 0.0f);
-      if (lead && v != 0.0f) atomic_add(p.dcolors + (size_t)id * p.C + ch, v);
-    }
+  for (int ch = 0; ch < p.C; ch++) {
+    const float v = wave_sum(px.inside ? wcol * dpix[(size_t)ch * HW] : 0.0f);
+    if (lead && v != 0.0f) atomic_add(p.dcolors + (size_t)id * p.C + ch, v);
   }
 #pragma unroll
   for (int r = 0; r < 2; r++) {
@@ -701,8 +940,6 @@ __device__ __forceinline__ void bwd_splat_sums(const RenderBwdParams& p, const B
   }
 }
 
-// Colour path (no grid): the wave walks the staged splats back to front in
-// lockstep, every lane one pixel.
 __global__ void __launch_bounds__(kBwdThreads) render_backward_colour_kernel(const RenderBwdParams p) {
   __shared__ float4 srec[4][kBwdThreads];
   __shared__ uint32_t sid[kBwdThreads];
@@ -747,23 +984,35 @@ __global__ void __launch_bounds__(kBwdThreads) render_backward_colour_kernel(con
         const float dxyz[3] = {0.0f, 0.0f, 0.0f};
         bwd_hit_grad<false>(px, h, q1, q2, q3, q3, q3, p.beta, contributor, dot, dxyz, gr, p.kernel_type);
       }
-      if (__ballot(act) != 0ull) bwd_splat_sums<false, 0>(p, px, id, act, gr, 0.0f, wcol, 0.0f, 0.0f);
+      if (__ballot(act) != 0ull) bwd_splat_sums(p, px, id, gr, wcol);
     }
   }
 }
 
-// Grid path.  A wave walks a batch of staged splats in segments of three
-// passes:
-//  1. geometry: the splats in lockstep, every lane one pixel; a hit with grid
-//     levels queues (grid coordinate, weight, grad_scale, owner lane, level
-//     count) in the wave's LDS queue, and every splat with a hit in the wave
-//     is listed with its hit and queue masks.  The segment ends when the
-//     queue could overflow at the next splat;
+// Grid path.  A wave walks a batch of staged splats back to front in segments
+// of three passes:
+//  1. hits: the splats whose bbox meets the wave's block one after the other,
+//     every lane one pixel; a hit takes a slot of the wave's LDS queue
+//     (intersection point, weight, owner lane, level count, 0 levels outside
+//     the grid) and is noted in its lane's list.  The queue is in splat order:
+//     hits of one splat share cells, and the table gradient, bound by its
+//     atomic requests, merges per cell (queued lane by lane instead, the 1M-splat
+//     frame sends 9.7e8 requests for 8.7e8).  The segment ends when the queue
+//     could overflow, some lane's list is full or the batch is through;
 //  2. grid: the queued hits spread one per lane, so the table gathers, the
 //     feature recomputation, dL/dxyz and the table-gradient scatter run with
 //     every lane busy; each hit's (dot, dxyz) replaces its queue entry;
-//  3. recursion: the listed splats again, in the same order, with the
-//     blending recursion per pixel and the per-splat wave sums.
+//  3. recursion: every lane works through its noted hits, in order (where few
+//     wide splats make up the segment, the wave goes splat by splat), with the
+//     blending recursion and the gradients into the batch's LDS sums.
+// Whole kernel, ms, lockstep walk / this: 150k splats, 801x517, 16 levels F=2
+// 22.3 / 20.3 (3.4e8 atomic requests, ~17 of the ~20 G/s random adds reach);
+// 1M splats, 1600x1064, F=4 54.6 / 50.8 (8.7e8 requests); 60k splats with
+// 24-float rows blended with 3 levels, 401x399, 10.1 / 7.1.
+// Frames of few tiles deal the levels round-robin over several workgroups per
+// tile (bwd_level_parts): everything the recursion sends out is linear in
+// (dot, dxyz) and the other loss terms, so each part sends its own levels'
+// share and part 0 the other terms.
 // kRows 1: render mode 4, per-splat feature rows (p.colors, p.pgd wide) ahead
 // of the grid's channels (CR/backward.cu:987-1040).  kRows 2: render mode 12
 // training, rows of p.cstride floats ending with the blend weight (p.wslot):
@@ -798,91 +1047,174 @@ __device__ __forceinline__ uint32_t bwd_hit_levels(const RenderBwdParams& p, con
 }
 
 constexpr int kBwdQueue = 256;  // queued grid hits per wave
-constexpr int kBwdList = 128;   // listed splats per wave and segment
-constexpr int kBwdWaves = kBwdThreads / 64;
+constexpr int kBwdBatch = 128;  // splats staged per batch
+constexpr int kBwdNoted = 8;    // hits a lane notes per segment
+constexpr uint32_t kBwdWideLanes = 16;  // lanes per splat from which they are
+constexpr int kBwdWide = 16;    // splats of a segment whose hits may be taken splat by splat
 
-// Three workgroups per CU (51.5 KB of LDS each) where the registers allow:
-// F <= 4 fits 168 VGPRs without spills, F = 8 keeps two.
+// A splat row's gradient on the leading n channels for the lanes with a hit,
+// coef * dL/dpixel_c (coefficient a below channel split, b from it on).  Lanes
+// at one splat, kBigGroup or more, are summed 32 channels at a time with a
+// reduce-scatter (as bwd_add_row) and added by consecutive lanes; the other
+// hits one at a time, lane c adding channel c of the hit's pixel, so that a hit
+// is one packed atomic per 64 channels.
+__device__ __forceinline__ void bwd_row_grads(const RenderBwdParams& p, bool on, uint32_t id, uint32_t stride, int n,
+                                              int split, float a, float b, const float* dpix) {
+  const size_t HW = (size_t)p.W * p.H;
+  const uint32_t off = on ? (uint32_t)(dpix - p.dL_dpix) : 0u;  // pixel index, below 2^31
+  const uint32_t lane = threadIdx.x & 63u;
+  uint64_t rem = __ballot(on);
+  while (rem != 0ull) {
+    const int ld = __ffsll((long long)rem) - 1;
+    const uint32_t hid = (uint32_t)__builtin_amdgcn_readlane((int)id, ld);
+    uint64_t m = __ballot(id == hid) & rem;
+    rem &= ~m;
+    float* row = p.dcolors + (size_t)hid * stride;
+    if ((uint32_t)__popcll(m) >= kBigGroup) {
+      const bool mem = ((m >> lane) & 1ull) != 0ull;
+      for (int c0 = 0; c0 < n; c0 += 32) {
+        const auto value = [&](int c) {
+          return mem && c < n ? (c < split ? a : b) * p.dL_dpix[(size_t)c * HW + off] : 0.0f;
+        };
+        float r[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) r[i] = halve(5, value(c0 + i), value(c0 + i + 16));
+        const int c = c0 + (int)reduce_scatter16(r);
+        if ((lane & 1u) == 0u && c < n) atomic_add(row + c, r[0]);
+      }
+      continue;
+    }
+    while (m != 0ull) {
+      const int l = __ffsll((long long)m) - 1;
+      m &= m - 1ull;
+      const float ha = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a), l));
+      const float hb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(b), l));
+      const uint32_t pix = (uint32_t)__builtin_amdgcn_readlane((int)off, l);
+      for (int c = (int)lane; c < n; c += 64) {
+        const float v = (c < split ? ha : hb) * p.dL_dpix[(size_t)c * HW + pix];
+        if (v != 0.0f) atomic_add(row + c, v);
+      }
+    }
+  }
+}
+
+// Three workgroups per CU (51.8 KB of LDS each) where the registers allow:
+// F <= 4 fits 168 VGPRs, F = 8 keeps two.
 template <int F, int kRows>
 __global__ void __launch_bounds__(kBwdThreads) __attribute__((amdgpu_waves_per_eu(F <= 4 ? 3 : 2)))
 render_backward_kernel(const RenderBwdParams p) {
-  __shared__ float4 srec[kBwdChunks][kBwdThreads];
-  __shared__ uint32_t sid[kBwdThreads];
+  constexpr int kMasks = kBwdBatch / 64;
+  __shared__ float4 srec[kBwdChunks][kBwdBatch];
+  __shared__ uint32_t sid[kBwdBatch];
+  __shared__ float sums[kBwdBatch * kSumHash];
   __shared__ float4 hq[kBwdWaves][kBwdQueue];       // (xyz, w), then (dot, dxyz)
   __shared__ uint16_t hmeta[kBwdWaves][kBwdQueue];  // owner lane | level count << 6
-  __shared__ uint64_t lact[kBwdWaves][kBwdList];
-  __shared__ uint8_t lj[kBwdWaves][kBwdList];
+  __shared__ uint16_t noted[kBwdNoted][kBwdThreads];  // batch index | queue slot << 8
+  __shared__ uint64_t lact[kBwdWaves][kBwdWide];      // the segment's first splats: lanes hit, batch index
+  __shared__ uint8_t lj[kBwdWaves][kBwdWide];
+  __shared__ uint64_t smask[kBwdWaves][kMasks];
 
-  const uint32_t tile = p.tile_order[blockIdx.x];  // the forward's order: heaviest tiles first
+  // level parts: workgroup b runs on XCD b % 8, dealt as in the forward
+  uint32_t pos = blockIdx.x, part = 0u;
+  if (p.parts > 1u) {
+    const uint32_t x = blockIdx.x % 8u, q = blockIdx.x / 8u;
+    part = x % p.parts;
+    pos = 8u * (q >> p.parts_log2) + x / p.parts + (8u >> p.parts_log2) * (q % p.parts);
+    if (pos >= p.ntiles) return;
+  }
+  const uint32_t tile = p.tile_order[pos];  // the forward's order: heaviest tiles first
   const uint2 range = reinterpret_cast<const uint2*>(p.ranges)[tile];
+  if (range.x >= range.y) return;
   const size_t HW = (size_t)p.W * p.H;
-  const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint64_t lt = lane == 0u ? 0ull : (~0ull >> (64u - lane));
   BwdPixel px;
   bwd_pixel_init(p, tile, px);
+  if (part != 0u) {
+    px.sum_abs = 0.0f;
+    px.dL_ddepth = px.dL_daccum = px.dL_dmedian = px.dL_dreg = 0.0f;
+    px.dn2[0] = px.dn2[1] = px.dn2[2] = 0.0f;
+  }
   const uint32_t tx = tile % p.gx, ty = tile / p.gx;
   const GridParams& g = p.grid;
   const nest_i32x4 rsrc = table_rsrc_rows<F, false>(g.table, g.table_rows);
   const size_t grid_ch = kRows ? (size_t)p.pgd * HW : 0;  // first grid channel of dL/dpixel
-
+  for (uint32_t i = threadIdx.x; i < kBwdBatch * kSumHash; i += kBwdThreads) sums[i] = 0.0f;
+  uint32_t* slast = reinterpret_cast<uint32_t*>(&hq[0][0]);  // the queues are empty yet
+  const uint32_t wlast = wave_max(px.last_contributor);
+  if (lane == 0u) slast[wid] = wlast;
+  __syncthreads();
   const uint32_t total = range.y - range.x;
-  for (uint32_t done_n = 0; done_n < total; done_n += kBwdThreads) {
-    const uint32_t n = min((uint32_t)kBwdThreads, total - done_n);
-    __syncthreads();
-    if (threadIdx.x < n) {
-      const uint32_t e = range.y - 1u - done_n - threadIdx.x;
-      const uint32_t id = p.point_list[e];
-      const float4* rec = reinterpret_cast<const float4*>(p.records) + 8 * (size_t)id;
+  const uint32_t tlast = min(total, max(max(slast[0], slast[1]), max(slast[2], slast[3])));
+
+  for (uint32_t below = tlast; below > 0u; below -= min(below, (uint32_t)kBwdBatch)) {
+    const uint32_t n = min((uint32_t)kBwdBatch, below);
+    if (threadIdx.x < (uint32_t)kBwdBatch) {
+      const bool in = threadIdx.x < n;
+      float4 bb = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (in) {
+        const uint32_t id = p.point_list[range.x + below - 1u - threadIdx.x];
+        const float4* rec = reinterpret_cast<const float4*>(p.records) + 8 * (size_t)id;
 #pragma unroll
-      for (int c = 0; c < kBwdChunks; c++) srec[c][threadIdx.x] = rec[c];
-      sid[threadIdx.x] = id;
+        for (int c = 0; c < kBwdChunks; c++) srec[c][threadIdx.x] = rec[c];
+        sid[threadIdx.x] = id;
+        bb = rec[7];
+      }
+      bwd_block_masks<kMasks>(in, bb, tx, ty, wid, smask);
     }
     __syncthreads();
-    for (uint32_t j0 = 0; j0 < n;) {
-      // 1. geometry
-      float T1 = px.T;
-      uint32_t cnt = 0, nl = 0, j = j0;
-      while (j < n) {
-        const uint32_t contributor = total - 1u - done_n - j;
-        const float4 q0 = srec[0][j], q1 = srec[1][j], q2 = srec[2][j];
+    uint64_t todo = 0ull;  // splats of the current 64 still to be visited
+    uint32_t chunk = 0u, j0 = 0u;
+    uint32_t qn = 0u, nn = 0u, nl = 0u;  // the wave's queued hits, the lane's noted ones, the wave's splats
+    float T1 = px.T;
+    for (;;) {
+      // 1. hits
+      bool segment = false;
+      while (!segment) {
+        if (todo == 0ull) {
+          if (chunk == (uint32_t)kMasks) break;
+          todo = wave_u64(smask[wid][chunk]);
+          j0 = chunk++ * 64u;
+          continue;
+        }
+        const uint32_t j = j0 + (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1ull;
+        const float4 q0 = srec[0][j], q1 = srec[1][j], q2 = srec[2][j], q6 = srec[6][j];
+        // the splat is number below - j of the tile's list, from 1
+        const bool near = below - j <= px.last_contributor && splat_near(q0, q1, q2, q6.y, px.pxf, px.pyf);
+        if (__ballot(near) == 0ull) continue;
         BwdHit h;
-        const bool act =
-            bwd_hit(q0, q1, q2, px.pxf, px.pyf, p.beta, px.inside && contributor < px.last_contributor, h,
-                    p.kernel_type, srec[6][j].z);
-        float xyz[3] = {0.0f, 0.0f, 0.0f}, hw = 0.0f;
-        uint32_t lane_levels = 0u;
+        const bool act = bwd_hit(q0, q1, q2, px.pxf, px.pyf, p.beta, near, h, p.kernel_type, q6.z);
+        const uint64_t m = __ballot(act);
+        if (m == 0ull) continue;
         if (act) {
           T1 = T1 / (1.f - h.alpha);
           const float wgt = h.alpha * T1;
-          float wt;
-          lane_levels = bwd_hit_levels<kRows>(p, h, srec[3][j], srec[4][j], srec[5][j], srec[6][j], sid[j], xyz, wt);
+          float wt, xyz[3];
+          const uint32_t lane_levels = bwd_hit_levels<kRows>(p, h, srec[3][j], srec[4][j], srec[5][j], q6, sid[j], xyz, wt);
           // the grid's share of the gradient: (1 - weight) of it in mode 12,
           // weight times it in mode 14
-          hw = kRows == 2 ? wgt * (p.azero ? wt : 1.0f - wt) : wgt;
-        }
-        const bool push = lane_levels > 0u;
-        const uint64_t m_act = __ballot(act), m_push = __ballot(push);
-        if (m_act != 0ull) {
-          if (lane == 0u) {
-            lact[wid][nl] = m_act;
-            lj[wid][nl] = (uint8_t)j;
-          }
-          nl++;
-        }
-        if (push) {
-          const uint32_t slot = cnt + (uint32_t)__popcll(m_push & lt);
+          const float hw = kRows == 2 ? wgt * (p.azero ? wt : 1.0f - wt) : wgt;
+          const uint32_t slot = qn + (uint32_t)__popcll(m & lt);
           hq[wid][slot] = make_float4(xyz[0], xyz[1], xyz[2], hw);
           hmeta[wid][slot] = (uint16_t)(lane | (lane_levels << 6));
+          noted[nn++][threadIdx.x] = (uint16_t)(j | slot << 8);
         }
-        cnt += (uint32_t)__popcll(m_push);
-        j++;
-        if (cnt > (uint32_t)(kBwdQueue - 64) || nl == (uint32_t)kBwdList) break;
+        if (nl < (uint32_t)kBwdWide && lane == 0u) {
+          lact[wid][nl] = m;
+          lj[wid][nl] = (uint8_t)j;
+        }
+        nl++;
+        qn += (uint32_t)__popcll(m);
+        segment = qn > (uint32_t)(kBwdQueue - 64) || __ballot(nn == (uint32_t)kBwdNoted) != 0ull;
       }
+      if (qn == 0u) break;  // the batch is through
       __builtin_amdgcn_wave_barrier();
       // 2. grid: table gradient, features' dot product and dL/dxyz per hit
-      for (uint32_t r0 = 0; r0 < cnt; r0 += 64u) {
+      for (uint32_t r0 = 0; r0 < qn; r0 += 64u) {
         const uint32_t e = r0 + lane;
-        const bool on = e < cnt;
+        const bool on = e < qn;
         float u[3] = {0.0f, 0.0f, 0.0f}, gsc = 0.0f, w = 0.0f;
         uint32_t lev = 0u;
         const float* dp = p.dL_dpix;
@@ -890,7 +1222,7 @@ render_backward_kernel(const RenderBwdParams p) {
           const float4 q = hq[wid][e];
           const float xyz[3] = {q.x, q.y, q.z};
           w = q.w;
-          grid_coord_bwd(g, xyz, u, gsc);  // inside the grid: the hit was queued
+          grid_coord_bwd(g, xyz, u, gsc);
           const uint32_t m = hmeta[wid][e];
           lev = m >> 6;
           const uint32_t t = (wid << 6) | (m & 63u);  // the owner's thread
@@ -900,54 +1232,60 @@ render_backward_kernel(const RenderBwdParams p) {
         // the chunk's queue entries (read above, rewritten below) stage the
         // table-gradient atomics meanwhile
         hash_backward_wave<F>(g, rsrc, u, gsc, lev, w, dp, HW, p.dtable, reinterpret_cast<uint32_t*>(&hq[wid][r0]),
-                              dot, dxyz);
+                              part, p.parts, dot, dxyz);
         if (on) hq[wid][e] = make_float4(dot, dxyz[0], dxyz[1], dxyz[2]);
       }
       __builtin_amdgcn_wave_barrier();
-      // 3. recursion and per-splat sums over the listed splats
-      uint32_t qbase = 0;
-      for (uint32_t i = 0; i < nl; i++) {
-        const uint32_t jj = lj[wid][i];
-        const uint64_t m_act = lact[wid][i];
-        const bool act = ((m_act >> lane) & 1ull) != 0ull;
-        const uint32_t contributor = total - 1u - done_n - jj;
-        const float4 q0 = srec[0][jj], q1 = srec[1][jj], q2 = srec[2][jj], q3 = srec[3][jj];
-        const float4 q4 = srec[4][jj], q5 = srec[5][jj];
-        const uint32_t id = sid[jj];
-        BwdHit h;
-        bwd_hit(q0, q1, q2, px.pxf, px.pyf, p.beta, act, h, p.kernel_type, srec[6][jj].z);
-        bool pushed = false;  // the hit's queue entry, as in the geometry pass
-        if (act) {
-          float xyz[3], wt0;
-          pushed = bwd_hit_levels<kRows>(p, h, q3, q4, q5, srec[6][jj], id, xyz, wt0) > 0u;
+      // 3. recursion and per-splat sums, over the noted hits or, where few wide
+      // splats make up the segment, splat by splat
+      const bool wide = nl <= (uint32_t)kBwdWide && qn >= nl * kBwdWideLanes;
+      uint32_t base = 0u;  // first queue slot of the splat
+      for (uint32_t i = 0; wide ? i < nl : __ballot(i < nn) != 0ull; i++) {
+        bool on = i < nn;
+        uint32_t e = 0u;
+        if (wide) {
+          const uint64_t m = lact[wid][i];
+          on = ((m >> lane) & 1ull) != 0ull;
+          e = lj[wid][i] | (base + (uint32_t)__popcll(m & lt)) << 8;
+          base += (uint32_t)__popcll(m);
+        } else if (on) {
+          e = noted[i][threadIdx.x];
         }
-        const uint64_t m_push = __ballot(pushed);
-        BwdGrad gr;
-        bwd_grad_zero(gr);
-        float gS = 0.0f, wcol = 0.0f, wt = 0.0f, fdot = 0.0f;
-        if (act) {
+        uint32_t id = 0u, j = 0u;
+        float wcol = 0.0f, wt = 0.0f;
+        float v[kSumHash];
+#pragma unroll
+        for (uint32_t k = 0; k < kSumHash; k++) v[k] = 0.0f;
+        if (on) {
+          j = e & 255u;
+          const float4 q1 = srec[1][j], q2 = srec[2][j], q3 = srec[3][j];
+          id = sid[j];
+          BwdHit h;
+          bwd_hit(srec[0][j], q1, q2, px.pxf, px.pyf, p.beta, true, h, p.kernel_type, srec[6][j].z);
           px.T = px.T / (1.f - h.alpha);
           const float wgt = h.alpha * px.T;
-          gS = wgt * px.sum_abs;
-          float rdot = 0.0f, dot = 0.0f, dxyz[3] = {0.0f, 0.0f, 0.0f};
-          if (pushed) {
-            const float4 r = hq[wid][qbase + (uint32_t)__popcll(m_push & lt)];
-            dot = r.x; dxyz[0] = r.y; dxyz[1] = r.z; dxyz[2] = r.w;
-          }
+          const float4 r = hq[wid][e >> 8];
+          float dot = r.x, fdot = 0.0f;
+          const float dxyz[3] = {r.y, r.z, r.w};
+          wcol = wgt;
           if constexpr (kRows == 1) {
-            const float* row = p.colors + (size_t)id * p.pgd;
-            for (int ch = 0; ch < p.pgd; ch++) rdot += row[ch] * px.dpix[(size_t)ch * HW];
-            wcol = wgt;
-            dot += rdot;
+            if (part == 0u) {
+              const float* row = p.colors + (size_t)id * p.pgd;
+              float rdot = 0.0f;
+              for (int ch = 0; ch < p.pgd; ch++) rdot += row[ch] * px.dpix[(size_t)ch * HW];
+              dot += rdot;
+            }
           } else if constexpr (kRows == 2) {
             // dot is grid . dpix over the fine channels; the hit's features are
             // the coarse rows and weight * row + (1 - weight) * grid
             const float* row = p.colors + (size_t)id * (uint32_t)p.cstride;
+            float rdot = 0.0f;
             wt = row[p.wslot];
-            for (int ch = 0; ch < p.pgd; ch++) rdot += row[ch] * px.dpix[(size_t)ch * HW];
-            if (!p.azero)
-              for (int i2 = 0; i2 < p.nfine; i2++) fdot += row[p.pgd + i2] * px.dpix[(size_t)(p.pgd + i2) * HW];
-            wcol = wgt;
+            if (part == 0u) {
+              for (int ch = 0; ch < p.pgd; ch++) rdot += row[ch] * px.dpix[(size_t)ch * HW];
+              if (!p.azero)
+                for (int i2 = 0; i2 < p.nfine; i2++) fdot += row[p.pgd + i2] * px.dpix[(size_t)(p.pgd + i2) * HW];
+            }
             const float hdot = dot;
             if (p.azero) {  // mode 14: coarse rows, then weight * grid
               dot = rdot + wt * hdot;
@@ -958,25 +1296,51 @@ render_backward_kernel(const RenderBwdParams p) {
               if (p.wsig) fdot = fdot * wt * (1.0f - wt);  // mode 7: dL/dlogit of weight = sigmoid(logit)
             }
           }
-          bwd_hit_grad<true>(px, h, q1, q2, q3, q4, q5, p.beta, contributor, dot, dxyz, gr, p.kernel_type);
+          BwdGrad gr;
+          bwd_grad_zero(gr);
+          bwd_hit_grad<true>(px, h, q1, q2, q3, srec[4][j], srec[5][j], p.beta, below - j - 1u, dot, dxyz, gr,
+                             p.kernel_type);
+          bwd_row_geometry(gr, v);
+#pragma unroll
+          for (uint32_t k = 0; k < 9; k++) v[kSumH + k] = gr.gH[k];
+          v[kSumS] = wgt * px.sum_abs;
+          v[kSumW] = fdot;
         }
-        qbase += (uint32_t)__popcll(m_push);
-        bwd_splat_sums<true, kRows>(p, px, id, act, gr, gS, wcol, wt, fdot);
+        bwd_add_row<kSumHash>(on, j, v, sums);
+        if constexpr (kRows == 1) {
+          if (part == 0u) bwd_row_grads(p, on, id, (uint32_t)p.pgd, p.pgd, p.pgd, wcol, 0.0f, px.dpix);
+        }
+        if constexpr (kRows == 2) {
+          if (part == 0u)
+            bwd_row_grads(p, on, id, (uint32_t)p.cstride, p.pgd + (p.azero ? 0 : p.nfine), p.pgd, wcol, wcol * wt,
+                          px.dpix);
+        }
       }
       __builtin_amdgcn_wave_barrier();
-      j0 = j;
+      qn = nn = nl = 0u;
+      T1 = px.T;
     }
+    __syncthreads();
+    bwd_flush_geometry<kSumHash>(p, sums, n, sid);
+    bwd_flush<kSumHash, 9>(sums, kSumH, n, sid, p.dhomo, 9);
+    bwd_flush<kSumHash, 1>(sums, kSumS, n, sid, p.gradsum, 1);
+    if constexpr (kRows == 2) bwd_flush<kSumHash, 1>(sums, kSumW, n, sid, p.dcolors + p.wslot, (uint32_t)p.cstride);
+    __syncthreads();
   }
 }
 
 template <int F, int kRows = 0>
 hipError_t launch_bwd_one(const RenderBwdParams& p, hipStream_t s) {
-  hipLaunchKernelGGL((render_backward_kernel<F, kRows>), dim3(p.ntiles), dim3(kBwdThreads), 0, s, p);
+  const uint32_t blocks = p.parts > 1u ? (p.ntiles + 7u) / 8u * 8u * p.parts : p.ntiles;
+  hipLaunchKernelGGL((render_backward_kernel<F, kRows>), dim3(blocks), dim3(kBwdThreads), 0, s, p);
   return hipGetLastError();
 }
 
 hipError_t launch_bwd_colour(const RenderBwdParams& p, hipStream_t s) {
-  hipLaunchKernelGGL(render_backward_colour_kernel, dim3(p.ntiles), dim3(kBwdThreads), 0, s, p);
+  if (p.C == 3)
+    hipLaunchKernelGGL(render_backward_rgb_kernel, dim3(p.ntiles), dim3(kBwdThreads), 0, s, p);
+  else
+    hipLaunchKernelGGL(render_backward_colour_kernel, dim3(p.ntiles), dim3(kBwdThreads), 0, s, p);
   return hipGetLastError();
 }
 
@@ -1275,8 +1639,26 @@ hipError_t launch_grid_encode_backward(const GridEncodeBwdParams& p, hipStream_t
   return hipGetLastError();
 }
 
-hipError_t launch_render_backward(const RenderBwdParams& p, hipStream_t s) {
-  if (p.ntiles == 0) return hipSuccess;
+// Workgroups per tile of the grid path, each with every parts-th level: few
+// tiles leave the chip idle behind each wave's chain of hits, levels and
+// scatter steps.  Repeating the hit and recursion passes costs more than it
+// gives once the tiles fill the chip and the atomics bound the launch.  Whole
+// backward, ms with 1 / 2 / 4 / 8 parts, 16 levels: 64 tiles 8.3 / 4.6 / 2.7 /
+// 1.8; 256 tiles 4.21 / 2.48 / 1.68 / 1.92; 625 tiles 11.5 / 7.2 / 7.6 / 8.2;
+// 1683 tiles 21.9 / 20.5 / 20.9 / 22.9 and 26.7 / 23.9 / 24.1 / 28.0; 4056
+// tiles 39.8 / 38.9 / 44.3 and 41.9 / 43.3 / 56.3.  3 levels: 256 tiles 1.39 /
+// 1.07 / 1.04; 676 tiles with feature rows 6.8 / 6.9; 1683 tiles 6.9 / 9.4.
+static uint32_t bwd_level_parts(uint32_t tiles, uint32_t L) {
+  if (L > 8u) return tiles <= 96u ? 8u : tiles <= 400u ? 4u : tiles <= 2560u ? 2u : 1u;
+  if (L >= 4u) return tiles <= 320u ? 4u : tiles <= 768u ? 2u : 1u;
+  return L >= 2u && tiles <= 320u ? 2u : 1u;
+}
+
+hipError_t launch_render_backward(const RenderBwdParams& p0, hipStream_t s) {
+  if (p0.ntiles == 0) return hipSuccess;
+  RenderBwdParams p = p0;
+  p.parts = p.level != 0 ? bwd_level_parts(p.ntiles, p.grid.L) : 1u;
+  p.parts_log2 = (uint32_t)__builtin_ctz(p.parts);
   if (p.wslot >= 0) {
     switch (p.grid.F) {
       case 2: return launch_bwd_one<2, 2>(p, s);

@@ -246,6 +246,8 @@ struct RenderBwdParams {
   int nfine;                  // render modes 12, 14: grid channels after the coarse ones (levels * F)
   int kernel_type;            // 0 Gaussian, 1 beta, 2 flex, 3 general (shape in record[26])
   float* dshapes;             // [P] kernel types 1-3
+  uint32_t parts;             // workgroups per tile the grid levels are dealt over, set by launch_render_backward
+  uint32_t parts_log2;
   GridParams grid;
 };
 hipError_t launch_render_backward(const RenderBwdParams& p, hipStream_t s);

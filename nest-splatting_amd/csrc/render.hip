@@ -41,6 +41,7 @@
 #include "hashgrid.h"
 #include "nest_internal.h"
 #include "nest_math.h"
+#include "splat_near.h"
 
 namespace nest {
 
@@ -485,24 +486,6 @@ __device__ __forceinline__ float kernel_g(int kt, float rho, float shape) {
   const float power = -0.5f * pow_term;
   if (power > 0.0f) return -1.0f;
   return expf_ref(power);
-}
-
-// Conservative form of the test below, for the pass that lists a pixel's
-// candidates: an rcp-based rho3d within 1e-6 of the exact one, scaled down by
-// 1e-5, above the splat's cut and rho2d above it too means alpha < 1/255 in
-// the exact test.  False only for such pairs; NaNs are candidates.
-__device__ __forceinline__ bool splat_near(float4 q0, float4 q1, float4 q2, float cut, float pxf, float pyf) {
-  const float Tu0 = q0.x, Tu1 = q0.y, Tu2 = q0.z, Tv0 = q0.w;
-  const float Tv1 = q1.x, Tv2 = q1.y, Tw0 = q1.z, Tw1 = q1.w;
-  const float Tw2 = q2.x;
-  const float k0 = pxf * Tw0 - Tu0, k1 = pxf * Tw1 - Tu1, k2 = pxf * Tw2 - Tu2;
-  const float l0 = pyf * Tw0 - Tv0, l1 = pyf * Tw1 - Tv1, l2 = pyf * Tw2 - Tv2;
-  const float p0 = k1 * l2 - k2 * l1, p1 = k2 * l0 - k0 * l2, p2 = k0 * l1 - k1 * l0;
-  const float dx = q2.y - pxf, dy = q2.z - pyf;
-  const float rho2d = 2.0f * (dx * dx + dy * dy);
-  const float rc = __builtin_amdgcn_rcpf(p2);
-  const float sxa = p0 * rc, sya = p1 * rc;
-  return !((sxa * sxa + sya * sya) * 0.99999f > cut && rho2d > cut);
 }
 
 __device__ __forceinline__ bool splat_hit(float4 q0, float4 q1, float4 q2, float pxf, float pyf, float beta,

@@ -146,6 +146,36 @@ def test_backward_hash_parity(oracle, name):
     _compare(*_setup(oracle, sc, "hash"))
 
 
+# (path, W, H, L, F, log scale): tile counts on both sides of each line of the
+# backward's level-parts rule (96, 400 and 2560 tiles over 8 levels; 320 and
+# 768 below), level counts the parts do not divide, and on the 3-channel path
+# splats of a pixel and of many waves (few and many lanes at one splat), with
+# several batches per tile.  The wide frames' splats cover thousands of pixels
+# (a 50 degree view 6,401 pixels wide), so a coarse level's row or a splat's scale
+# sums up to n = 57,609 pixels x 11 hits = 6.3e5 terms of both signs, where TOL is
+# for a few thousand: a sequential float32 sum errs by about u sqrt(n) of its
+# largest partial sum, u sqrt(6.3e5) = 4.7e-5, on both sides: 1e-4 (measured:
+# 2.6e-5 with the lockstep kernel, 2.4e-5 with lists).
+EDGE_TOL = 1e-4
+EDGE_CASES = [("hash", 96 * 16, 16, 16, 2, -3.0), ("hash", 97 * 16 - 3, 13, 11, 4, -3.0),
+              ("hash", 401 * 16 - 15, 9, 16, 2, -3.0), ("hash", 2561 * 16, 5, 9, 1, -3.0),
+              ("hash", 321 * 16, 9, 5, 2, -3.0), ("hash", 769 * 16, 7, 8, 4, -3.0), ("hash", 40, 24, 2, 4, -2.0),
+              ("hash", 17, 33, 16, 2, -4.5), ("sh", 40, 24, 1, 2, -2.0), ("sh", 17, 33, 1, 2, -5.5),
+              ("sh", 400, 16, 1, 2, -3.5)]
+
+
+@pytest.mark.parametrize("path,W,H,L,F,ls", EDGE_CASES)
+def test_backward_edges_parity(oracle, path, W, H, L, F, ls):
+    from nest_splat.scene import get_spec, make_scene
+    print(f"[case] backward {path} {W}x{H} L={L} F={F} log scale {ls}", flush=True)
+    gpu, ref, pre = _setup(oracle, make_scene(get_spec("cfg2", name="edges", P=6000, W=W, H=H, L=L, F=F, log2T=15,
+                                                       log_scale_mu=ls)), path)
+    for k, r in ref.items():
+        assert np.isfinite(gpu[k]).all(), k
+        assert np.abs(gpu[k].astype(np.float64) - r).max() <= EDGE_TOL * np.abs(r).max(), k
+    assert np.abs(ref["dopacity"]).max() > 0
+
+
 @pytest.mark.parametrize("path,beta", [("colors", 0.0), ("sh", 0.0), ("colors", 1.5)])
 def test_backward_colour_parity(oracle, path, beta):
     sc = scene("shell_small")
