@@ -782,81 +782,170 @@ static hipError_t launch_mfma32(const MlpParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// float32 path on the vector ALU: one lane per pixel, weights in LDS, one
-// wave per workgroup so that a small image still spreads over every CU (a
-// 128x128 frame is 256 workgroups instead of 64).
-constexpr int kMlpF32Threads = 64;
+// float32 path on v_mfma_f32_16x16x4: binary32 products and sums, one wave per
+// 16 NJ pixels, Y^T = W X^T layer by layer as above.  An accumulator's
+// register i holds hidden unit 16 mt + 4 (lane / 16) + i of pixel lane % 16,
+// which is the next layer's B operand if its k-steps run over (mt, i), so
+// hidden activations stay in registers; a lane's A operands of four
+// consecutive k-steps are four consecutive weights of one row.  Input k is
+// 16 q + 4 (lane / 16) + i: the features padded with zeros to whole chunks of
+// 16, then the 16 SH terms.  Weights sit in LDS in operand order (float4 per
+// chunk, M-tile and lane: 16-byte reads without conflicts).
+//
+// Bound by the matrix units' binary32 rate: 640,000 pixels of 32 channels at
+// width 64 are 70 us of 32-cycle instructions and take 116 us.  One lane per
+// pixel on the vector ALU, every weight read from LDS for every pixel, took
+// 876 us.
+constexpr int kMlpF32Threads = 256;
 
-template <int NW>
+__device__ __forceinline__ f32x4 relu4(f32x4 v) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i] = fmaxf(v[i], 0.0f);
+  return v;
+}
+
+// kVec: pixel-major features whose rows are whole aligned float4s.
+template <int NT, int NJ, bool kVec>
 __global__ void __launch_bounds__(kMlpF32Threads) mlp_f32_kernel(const MlpParams p) {
-  extern __shared__ float wl[];
-  const int C = p.C, Kin = C + 16;
-  float* w1 = wl;
-  float* w2 = w1 + NW * Kin;
-  float* w3 = w2 + NW * NW;
+  extern __shared__ float4 wl[];
+  const int C = p.C, Kin = C + 16, QF = (C + 15) / 16;
+  constexpr int W = 16 * NT;
+  float4* w1 = wl;                        // [QF + 1][NT][64]
+  float4* w2 = w1 + (QF + 1) * NT * 64;   // [NT][NT][64]
+  float4* w3 = w2 + NT * NT * 64;         // [NT][64]: rows 0-2 of 16
   const float* g1 = static_cast<const float*>(p.w1);
   const float* g2 = static_cast<const float*>(p.w2);
   const float* g3 = static_cast<const float*>(p.w3);
-  // W1 transposed to [k][j]: a feature's NW weights are one contiguous run,
-  // read four at a time
-  for (int i = threadIdx.x; i < NW * Kin; i += kMlpF32Threads) w1[(i % Kin) * NW + i / Kin] = g1[i];
-  for (int i = threadIdx.x; i < NW * NW; i += kMlpF32Threads) w2[i] = g2[i];
-  for (int i = threadIdx.x; i < 3 * NW; i += kMlpF32Threads) w3[i] = g3[i];
+  for (int e = threadIdx.x; e < (QF + 1) * NT * 64; e += kMlpF32Threads) {
+    const int l = e & 63, t = e >> 6, q = t / NT, k = 4 * (l >> 4);
+    const float* row = g1 + (size_t)(16 * (t - q * NT) + (l & 15)) * Kin;
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int c = q < QF ? 16 * q + k + i : C + k + i;
+      v[i] = q < QF && c >= C ? 0.0f : row[c];
+    }
+    w1[e] = make_float4(v[0], v[1], v[2], v[3]);
+  }
+  for (int e = threadIdx.x; e < NT * NT * 64; e += kMlpF32Threads) {
+    const int l = e & 63, t = e >> 6, q = t / NT;
+    const float* r = g2 + (16 * (t - q * NT) + (l & 15)) * W + 16 * q + 4 * (l >> 4);
+    w2[e] = make_float4(r[0], r[1], r[2], r[3]);
+  }
+  for (int e = threadIdx.x; e < NT * 64; e += kMlpF32Threads) {
+    const int l = e & 63, q = e >> 6;
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if ((l & 15) < 3) {
+      const float* r = g3 + (l & 15) * W + 16 * q + 4 * (l >> 4);
+      v = make_float4(r[0], r[1], r[2], r[3]);
+    }
+    w3[e] = v;
+  }
   __syncthreads();
-  for (int64_t n = (int64_t)blockIdx.x * kMlpF32Threads + threadIdx.x; n < p.N; n += (int64_t)gridDim.x * kMlpF32Threads) {
-    float dx, dy, dz;
-    pixel_dir(p, n, dx, dy, dz);
-    float sh[16];
-    sh16(dx, dy, dz, sh);
-    float h1[NW];
+  const int lane = (int)(threadIdx.x & 63u), col = lane & 15, grp = lane >> 4;
+  const int64_t step = (int64_t)gridDim.x * (kMlpF32Threads / 64) * (16 * NJ);
+  for (int64_t n0 = ((int64_t)blockIdx.x * (kMlpF32Threads / 64) + (threadIdx.x >> 6)) * (16 * NJ); n0 < p.N; n0 += step) {
+    int64_t n[NJ];
 #pragma unroll
-    for (int j = 0; j < NW; j++) h1[j] = 0.0f;
-    for (int k = 0; k < C; k++) {
-      const float xk = p.feat[(int64_t)k * p.feat_cs + n * p.feat_ns];
-      const float4* wk = reinterpret_cast<const float4*>(w1 + k * NW);
+    for (int j = 0; j < NJ; j++) n[j] = min(n0 + 16 * j + col, p.N - 1);
+    f32x4 a1[NT][NJ];
 #pragma unroll
-      for (int j = 0; j < NW / 4; j++) {
-        const float4 w = wk[j];
-        h1[4 * j] += w.x * xk;
-        h1[4 * j + 1] += w.y * xk;
-        h1[4 * j + 2] += w.z * xk;
-        h1[4 * j + 3] += w.w * xk;
+    for (int mt = 0; mt < NT; mt++)
+#pragma unroll
+      for (int j = 0; j < NJ; j++) a1[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the view direction's terms first: the features' loads are in flight
+    float x[2][NJ][4];
+    const auto load = [&](int q, float (&v)[NJ][4]) {
+      const int c = 16 * q + 4 * grp;
+#pragma unroll
+      for (int j = 0; j < NJ; j++) {
+        const float* f = p.feat + n[j] * p.feat_ns;
+        if constexpr (kVec) {
+          const float4 r = c < C ? *reinterpret_cast<const float4*>(f + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+          v[j][0] = r.x; v[j][1] = r.y; v[j][2] = r.z; v[j][3] = r.w;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; i++) v[j][i] = c + i < C ? f[(int64_t)(c + i) * p.feat_cs] : 0.0f;
+        }
+      }
+    };
+    const auto layer1 = [&](int q, const float (&v)[NJ][4]) {
+#pragma unroll
+      for (int mt = 0; mt < NT; mt++) {
+        const float4 a = w1[(q * NT + mt) * 64 + lane];
+        const float av[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int j = 0; j < NJ; j++)
+            a1[mt][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], v[j][i], a1[mt][j], 0, 0, 0);
+      }
+    };
+    load(0, x[0]);
+    float sx[NJ][4];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+      float dx, dy, dz, sh[16];
+      pixel_dir(p, n[j], dx, dy, dz);
+      sh16(dx, dy, dz, sh);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float lo = (grp & 1) ? sh[4 + i] : sh[i], hi = (grp & 1) ? sh[12 + i] : sh[8 + i];
+        sx[j][i] = (grp & 2) ? hi : lo;
       }
     }
+    for (int q = 0; q < QF; q += 2) {
+      if (q + 1 < QF) load(q + 1, x[1]);
+      layer1(q, x[0]);
+      if (q + 2 < QF) load(q + 2, x[0]);
+      if (q + 1 < QF) layer1(q + 1, x[1]);
+    }
+    layer1(QF, sx);
+    f32x4 a2[NT][NJ];
 #pragma unroll
-    for (int s = 0; s < 16; s++) {
-      const float4* wk = reinterpret_cast<const float4*>(w1 + (C + s) * NW);
+    for (int mt = 0; mt < NT; mt++)
 #pragma unroll
-      for (int j = 0; j < NW / 4; j++) {
-        const float4 w = wk[j];
-        h1[4 * j] += w.x * sh[s];
-        h1[4 * j + 1] += w.y * sh[s];
-        h1[4 * j + 2] += w.z * sh[s];
-        h1[4 * j + 3] += w.w * sh[s];
+      for (int j = 0; j < NJ; j++) a2[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < NT; q++) {
+#pragma unroll
+      for (int j = 0; j < NJ; j++) a1[q][j] = relu4(a1[q][j]);
+#pragma unroll
+      for (int mt = 0; mt < NT; mt++) {
+        const float4 a = w2[(q * NT + mt) * 64 + lane];
+        const float av[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int j = 0; j < NJ; j++)
+            a2[mt][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], a1[q][j][i], a2[mt][j], 0, 0, 0);
       }
     }
+    f32x4 a3[NJ];
 #pragma unroll
-    for (int j = 0; j < NW; j++) h1[j] = fmaxf(h1[j], 0.0f);
-    float o0 = 0.f, o1 = 0.f, o2 = 0.f;
-    for (int j = 0; j < NW; j++) {
-      float h = 0.0f;
-      const float4* wj = reinterpret_cast<const float4*>(w2 + j * NW);
+    for (int j = 0; j < NJ; j++) a3[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int k = 0; k < NW / 4; k++) {
-        const float4 w = wj[k];
-        h += w.x * h1[4 * k];
-        h += w.y * h1[4 * k + 1];
-        h += w.z * h1[4 * k + 2];
-        h += w.w * h1[4 * k + 3];
-      }
-      h = fmaxf(h, 0.0f);
-      o0 += w3[j] * h;
-      o1 += w3[NW + j] * h;
-      o2 += w3[2 * NW + j] * h;
+    for (int q = 0; q < NT; q++) {
+      const float4 a = w3[q * 64 + lane];
+      const float av[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+      for (int j = 0; j < NJ; j++) a2[q][j] = relu4(a2[q][j]);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+          a3[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], a2[q][j][i], a3[j], 0, 0, 0);
     }
-    p.out[0 * p.out_os + n * p.out_ns] = finish_rgb(p, n, o0, 0);
-    p.out[1 * p.out_os + n * p.out_ns] = finish_rgb(p, n, o1, 1);
-    p.out[2 * p.out_os + n * p.out_ns] = finish_rgb(p, n, o2, 2);
+    if (grp == 0) {
+#pragma unroll
+      for (int j = 0; j < NJ; j++) {
+        const int64_t m = n0 + 16 * j + col;
+        if (m < p.N) {
+#pragma unroll
+          for (int o = 0; o < 3; o++) p.out[o * p.out_os + m * p.out_ns] = finish_rgb(p, m, a3[j][o], o);
+        }
+      }
+    }
   }
 }
 
@@ -884,13 +973,27 @@ static hipError_t launch_mfma(const MlpParams& p, hipStream_t s) {
   }
 }
 
-template <int NW>
-static hipError_t launch_f32(const MlpParams& p, hipStream_t s) {
-  const size_t lds = sizeof(float) * ((size_t)NW * (p.C + 16) + (size_t)NW * NW + 3 * (size_t)NW);
-  const int64_t want = (p.N + kMlpF32Threads - 1) / kMlpF32Threads;
-  const unsigned blocks = (unsigned)(want < 8192 ? (want > 0 ? want : 1) : 8192);
-  hipLaunchKernelGGL(mlp_f32_kernel<NW>, dim3(blocks), dim3(kMlpF32Threads), lds, s, p);
+template <int NT, int NJ>
+static hipError_t launch_f32_tiles(const MlpParams& p, hipStream_t s) {
+  const int QF = (p.C + 15) / 16;
+  const size_t lds = sizeof(float4) * 64 * (size_t)((QF + 1) * NT + NT * NT + NT);
+  const int64_t per = 16 * NJ * (kMlpF32Threads / 64);
+  const int64_t want = (p.N + per - 1) / per;
+  const unsigned blocks = (unsigned)(want < 1024 ? want : 1024);
+  const bool vec = p.feat_cs == 1 && p.C % 4 == 0 && p.feat_ns % 4 == 0 && (reinterpret_cast<uintptr_t>(p.feat) & 15u) == 0;
+  if (vec)
+    hipLaunchKernelGGL((mlp_f32_kernel<NT, NJ, true>), dim3(blocks), dim3(kMlpF32Threads), lds, s, p);
+  else
+    hipLaunchKernelGGL((mlp_f32_kernel<NT, NJ, false>), dim3(blocks), dim3(kMlpF32Threads), lds, s, p);
   return hipGetLastError();
+}
+
+// One 16-pixel tile per wave while that leaves at most two waves on a SIMD
+// (a 128x128 frame is 256 workgroups), two tiles sharing their weight reads
+// beyond.
+template <int NT>
+static hipError_t launch_f32(const MlpParams& p, hipStream_t s) {
+  return p.N <= 32768 ? launch_f32_tiles<NT, 1>(p, s) : launch_f32_tiles<NT, 2>(p, s);
 }
 
 template <bool kBF16>
@@ -919,9 +1022,9 @@ hipError_t launch_mlp(const MlpParams& p, hipStream_t s) {
   if (p.N <= 0) return hipSuccess;
   if (p.dtype == NEST_DTYPE_F32) {
     switch (p.width) {
-      case 16: return launch_f32<16>(p, s);
-      case 32: return launch_f32<32>(p, s);
-      case 64: return launch_f32<64>(p, s);
+      case 16: return launch_f32<1>(p, s);
+      case 32: return launch_f32<2>(p, s);
+      case 64: return launch_f32<4>(p, s);
       default: return hipErrorInvalidValue;
     }
   }

@@ -4,8 +4,8 @@
 NestMLP holds the bias-free weights of the reference's network
 (n_input = C + 16 -> width -> width -> 3, ReLU hidden, sigmoid output) as
 float32 parameters plus cached copies in the compute dtype, and runs them on
-libnest_splat: MFMA (v_mfma_f32_16x16x16 f16/bf16) for float16/bfloat16, the
-vector ALU for float32.  The SphericalHarmonics degree-4 view encoding and the
+libnest_splat: MFMA for every type (v_mfma_f32_16x16x16 and x32 f16/bf16,
+v_mfma_f32_16x16x4 for float32).  The SphericalHarmonics degree-4 view encoding and the
 (d+1)/2 input mapping are fused into the kernel.
 """
 from __future__ import annotations

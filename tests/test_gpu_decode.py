@@ -36,6 +36,36 @@ def test_mlp_rgb_decode(oracle, C, width, dtype, N):
     tol = 1e-5 if dtype == "f32" else 1e-3
     np.testing.assert_allclose(out, ref, atol=tol, rtol=0)
 
+@pytest.mark.parametrize("C,width,N", [(1, 16, 1), (10, 64, 15), (16, 32, 17), (20, 64, 129), (40, 16, 1000),
+                                       (48, 64, 32768), (32, 64, 32769), (128, 64, 40001)])
+@pytest.mark.parametrize("layout", ["rows", "odd rows", "planes"])
+def test_mlp_f32_tiles(C, width, N, layout):
+    """The float32 MLP's chunks of 16 inputs (whole, padded, many), its one-
+    and two-tile waves and ragged ends, over feature rows that are whole
+    aligned float4s, rows that are not, and channel planes, against the
+    network in 64 bits.  A logit is three chained sums of at most 144, 64 and
+    64 products with |x| below ~1.5 and |w| below 1: within 144 * 2^-24 of
+    values of a few units, and the sigmoid's slope is at most 1/4: 1e-5."""
+    from nest_splat.mlp import NestMLP
+    g = torch.Generator(device=DEV).manual_seed(C * 1000 + N)
+    pad = C + 3 if layout == "odd rows" else C
+    feat = torch.randn((N, pad), generator=g, device=DEV)[:, :C] * 0.3
+    if layout == "planes":
+        feat = feat.t().contiguous().t()
+    dirs = torch.nn.functional.normalize(torch.randn((N, 3), generator=g, device=DEV), dim=1)
+    m = NestMLP(C, width, "f32", seed=7).to(DEV)
+    out = m.rgb_decode(feat, dirs).double()
+    x, y, z = dirs.double().unbind(1)
+    sh = [0.28209479177387814 + 0 * x, -0.48860251190291987 * y, 0.48860251190291987 * z, -0.48860251190291987 * x,
+          1.0925484305920792 * x * y, -1.0925484305920792 * y * z, 0.94617469575755997 * z * z - 0.31539156525251999,
+          -1.0925484305920792 * x * z, 0.54627421529603959 * (x * x - y * y), 0.59004358992664352 * y * (y * y - 3 * x * x),
+          2.8906114426405538 * x * y * z, 0.45704579946446572 * y * (1 - 5 * z * z), 0.3731763325901154 * z * (5 * z * z - 3),
+          0.45704579946446572 * x * (1 - 5 * z * z), 1.4453057213202769 * z * (x * x - y * y),
+          0.59004358992664352 * x * (3 * y * y - x * x)]
+    h = torch.cat([feat.double(), torch.stack(sh, 1)], 1)
+    h = torch.relu(torch.relu(h @ m.W1.double().t()) @ m.W2.double().t()) @ m.W3.double().t()
+    assert (out - torch.sigmoid(h)).abs().max().item() <= 1e-5
+
 
 def test_mlp_strided_features_and_mask(oracle):
     """rgb_decode on the channel-major permuted view (no copy), with the
