@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NEST_ABI_VERSION 17
+#define NEST_ABI_VERSION 18
 
 #define NEST_OK 0
 #define NEST_ERR_INVALID_ARGUMENT (-1)
@@ -438,6 +438,20 @@ int nest_backward(const nest_raster_settings *settings, const nest_hashgrid *gri
  * reference's float32 expressions. */
 int nest_build_homotrans(int64_t P, const float *rotations, const float *scales, const float *means3D,
                          float *homotrans, void *stream);
+
+/* Surface maps of a frame (gaussian_renderer/__init__.py:763-791,
+ * utils/point_utils.py:10-60) from its allmap [>= 7][H][W]: the world-space
+ * normal map (view_rotation: row-major 3x3, normal_c = sum_k
+ * view_rotation[3 c + k] allmap[2 + k]), expected depth allmap[0] / allmap[1]
+ * and median depth allmap[5] (NaN and +inf as 0), their blend expected_share *
+ * expected + median_share * median, and the normal of the blended depth map
+ * back-projected along the rays (x, y, 1) @ ray_matrix from origin, times
+ * alpha.  The normal maps are [H][W][3], the depths [H][W]; device float32
+ * arrays, the matrices and origin host arrays; W * H below 2^31. */
+int nest_surface_maps(int32_t W, int32_t H, const float *allmap, const float view_rotation[9],
+                      const float ray_matrix[9], const float origin[3], float expected_share, float median_share,
+                      float *rend_normal, float *surf_depth, float *surf_normal, float *depth_expected,
+                      float *depth_median, void *stream);
 
 /* markVisible (DSR/rasterize_points.cu:452-470, CR/rasterizer_impl.cu:198-210,
  * checkFrustum :54-66): present[i] = 1 when the view-space depth of

@@ -24,7 +24,7 @@ OUT = os.path.join(HERE, "nest_splat", "libnest_splat.so")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 
 SOURCES = ["abi.cpp", "preprocess.hip", "binning.hip", "render.hip", "backward.hip", "grid_encode.hip", "mlp.hip",
-           "rvq.hip"]
+           "rvq.hip", "surface.hip"]
 
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 ARCH = os.environ.get("NEST_OFFLOAD_ARCH", "gfx950")

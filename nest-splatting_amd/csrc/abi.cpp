@@ -792,6 +792,34 @@ int nest_forward_render(const nest_raster_settings* rs, const nest_hashgrid* gr,
   return NEST_OK;
 }
 
+int nest_surface_maps(int32_t W, int32_t H, const float* allmap, const float view_rotation[9],
+                      const float ray_matrix[9], const float origin[3], float expected_share, float median_share,
+                      float* rend_normal, float* surf_depth, float* surf_normal, float* depth_expected,
+                      float* depth_median, void* stream) {
+  if (W < 0 || H < 0) return fail(NEST_ERR_INVALID_ARGUMENT, "W and H must be >= 0 (got %d x %d)", W, H);
+  if ((int64_t)W * H >= (1ll << 31)) return fail(NEST_ERR_UNSUPPORTED, "surface maps take fewer than 2^31 pixels");
+  if (W == 0 || H == 0) return NEST_OK;
+  if (!allmap || !view_rotation || !ray_matrix || !origin || !rend_normal || !surf_depth || !surf_normal ||
+      !depth_expected || !depth_median)
+    return fail(NEST_ERR_INVALID_ARGUMENT, "NULL pointer");
+  SurfaceParams p{};
+  p.W = W;
+  p.H = H;
+  p.allmap = allmap;
+  memcpy(p.R, view_rotation, sizeof(p.R));
+  memcpy(p.M, ray_matrix, sizeof(p.M));
+  memcpy(p.origin, origin, sizeof(p.origin));
+  p.expected_share = expected_share;
+  p.median_share = median_share;
+  p.rend_normal = rend_normal;
+  p.surf_depth = surf_depth;
+  p.surf_normal = surf_normal;
+  p.depth_expected = depth_expected;
+  p.depth_median = depth_median;
+  hipError_t e = launch_surface(p, static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? NEST_OK : hip_fail(e, "surface_maps");
+}
+
 int nest_build_homotrans(int64_t P, const float* rotations, const float* scales, const float* means3D,
                          float* homotrans, void* stream) {
   if (P < 0) return fail(NEST_ERR_INVALID_ARGUMENT, "P must be >= 0 (got %lld)", (long long)P);

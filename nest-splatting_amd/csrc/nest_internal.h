@@ -350,6 +350,22 @@ struct MlpParams {
 };
 hipError_t launch_mlp(const MlpParams& p, hipStream_t s);
 
+// Surface maps of a frame (nest_surface_maps).
+struct SurfaceParams {
+  int W, H;
+  const float* allmap;    // [14][H][W]
+  float R[9];             // rend_normal_c = sum_k R[3 c + k] normal_k
+  float M[9];             // ray of pixel (x, y): (x, y, 1) @ M
+  float origin[3];
+  float expected_share, median_share;  // of the blended depth
+  float* rend_normal;     // [H][W][3]
+  float* surf_depth;      // [H][W]
+  float* surf_normal;     // [H][W][3]
+  float* depth_expected;  // [H][W]
+  float* depth_median;    // [H][W]
+};
+hipError_t launch_surface(const SurfaceParams& p, hipStream_t s);
+
 struct RvqParams {
   int64_t P;
   int stages;

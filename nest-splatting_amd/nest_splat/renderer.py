@@ -20,6 +20,7 @@ raw SH colours or the SH coefficients to render modes 8-10 with a one-level
 """
 from __future__ import annotations
 
+import ctypes as ct
 import math
 from dataclasses import dataclass
 from typing import Optional
@@ -28,6 +29,7 @@ import numpy as np
 import torch
 import torch.nn.functional as torch_F
 
+from . import _lib as L
 from . import rasterizer as rz
 from .camera import Camera, view_ray_matrix
 from .mlp import NestMLP
@@ -441,11 +443,46 @@ def _render_hybrid(cam, pc, pipe, bg_color, scaling_modifier, ingp, beta, max_in
     return rets
 
 
+def _plain_map(t: torch.Tensor) -> bool:
+    """Whether a map can go to a kernel as memory: an ordinary contiguous
+    float32 device tensor that no gradient, transform, mode or trace follows."""
+    if type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.float32 or not t.is_contiguous():
+        return False
+    if t.ndim != 3 or t.shape[0] < 8 or t.shape[1] * t.shape[2] >= 1 << 31 or (torch.is_grad_enabled() and t.requires_grad):
+        return False
+    return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None and
+            torch._C._len_torch_dispatch_stack() == 0 and not torch._C._is_torch_function_mode_enabled() and
+            not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+
+
+def _surface_maps_fused(cam, allmap: torch.Tensor, depth_ratio: float) -> dict:
+    """surface_maps in one kernel (nest_surface_maps)."""
+    H, W = int(allmap.shape[1]), int(allmap.shape[2])
+    if (H, W) != (cam.image_height, cam.image_width):
+        raise ValueError(f"allmap is {H} x {W}, the camera {cam.image_height} x {cam.image_width}")
+    normals = torch.empty((2, H, W, 3), dtype=torch.float32, device=allmap.device)
+    depths = torch.empty((3, 1, H, W), dtype=torch.float32, device=allmap.device)
+    wv = cam.world_view_transform
+    wv = wv.detach().cpu().numpy() if isinstance(wv, torch.Tensor) else np.asarray(wv)
+    f9 = ct.c_float * 9
+    R = f9(*wv[:3, :3].astype(np.float32).reshape(-1).tolist())
+    M = f9(*view_ray_matrix(cam).reshape(-1).tolist())
+    origin = (ct.c_float * 3)(*np.linalg.inv(wv.astype(np.float64).T)[:3, 3].tolist())
+    L.check(L.lib().nest_surface_maps(W, H, L.ptr(allmap), R, M, origin, 1 - depth_ratio, depth_ratio,
+                                      L.ptr(normals[0]), L.ptr(depths[0]), L.ptr(normals[1]), L.ptr(depths[1]),
+                                      L.ptr(depths[2]), L.stream_ptr(allmap.device)), "nest_surface_maps")
+    return {"rend_alpha": allmap[1:2], "rend_normal": normals[0].permute(2, 0, 1), "rend_dist": allmap[6:7],
+            "surf_depth": depths[0], "surf_normal": normals[1].permute(2, 0, 1), "gaussian_num": allmap[7:8],
+            "depth_expected": depths[1], "depth_median": depths[2]}
+
+
 def surface_maps(cam, allmap: torch.Tensor, depth_ratio: float = 0.0) -> dict:
     """The allmap post-processing of gaussian_renderer/__init__.py:763-791:
     world-space normal map, median and expected depth, distortion, the
     pseudo-surface depth (depth_ratio blends expected and median depth) and
     its normal from the back-projected depth map, scaled by alpha."""
+    if _plain_map(allmap) and type(depth_ratio) in (int, float):
+        return _surface_maps_fused(cam, allmap, depth_ratio)
     dev = allmap.device
     render_alpha = allmap[1:2]
     wv = _matrix(cam.world_view_transform, dev)

@@ -1,0 +1,69 @@
+"""GPU parity of the fused surface maps (nest_surface_maps) against the same
+expressions as tensor operations on the CPU."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _allmap(W, H, seed):
+    """A wavy surface at depth ~3 with every kind of depth: none (alpha 0,
+    depth 0), infinite and NaN."""
+    g = torch.Generator().manual_seed(seed)
+    y, x = torch.meshgrid(torch.arange(H).float(), torch.arange(W).float(), indexing="ij")
+    a = torch.rand((14, H, W), generator=g)
+    a[1] = 0.3 + 0.7 * a[1]
+    a[0] = (3 + 0.3 * torch.sin(x / 7) + 0.2 * torch.cos(y / 5)) * a[1]
+    a[5] = a[0] / a[1] + 0.01
+    if W * H > 8:
+        a[0:2, H // 2, W // 3:] = 0.0
+        a[0, 0, 0], a[1, 0, 0] = 1.0, 0.0
+        a[5, H - 1, W // 2] = float("nan")
+        a[5, H // 3, W - 1] = float("-inf")
+    return a
+
+
+@pytest.mark.parametrize("W,H", [(1, 1), (2, 5), (3, 3), (64, 4), (97, 61)])
+@pytest.mark.parametrize("ratio", [0.0, 0.3, 1])
+def test_surface_maps_fused(W, H, ratio):
+    """Depths bit for bit.  Points are within ~1e-6 of coordinates of ~3
+    (binary32 products and sums in another order), their differences over two
+    pixels at least ~0.03 long, so the normals within 1e-4."""
+    from nest_splat.camera import look_at
+    from nest_splat.renderer import surface_maps
+    cam = look_at((0.4, -3.0, 1.0), (0, 0, 0), 50.0, W, H)
+    a = _allmap(W, H, W + H)
+    ref = surface_maps(cam, a, ratio)
+    dev = a.to(DEV)
+    out = surface_maps(cam, dev, ratio)
+    assert set(out) == set(ref)
+    for k, v in ref.items():
+        o = out[k].cpu()
+        assert o.shape == v.shape and out[k].stride() == v.stride(), k
+        if k == "rend_normal":
+            np.testing.assert_allclose(o.numpy(), v.numpy(), atol=1e-6)
+        elif k == "surf_normal":
+            big = (ref["surf_depth"].abs() > 1e30)  # -inf became the lowest finite: its neighbours overflow
+            near = torch.nn.functional.max_pool2d(big.float(), 3, 1, 1)[0] > 0
+            keep = ~near.expand_as(v)
+            np.testing.assert_allclose(o[keep].numpy(), v[keep].numpy(), atol=1e-4)
+        else:
+            np.testing.assert_array_equal(o.numpy(), v.numpy(), err_msg=k)
+
+
+def test_surface_maps_gradient_and_views_keep_the_general_path():
+    """A map that gradients follow, and one that is not contiguous."""
+    from nest_splat.camera import look_at
+    from nest_splat.renderer import surface_maps
+    W, H = 33, 20
+    cam = look_at((0.4, -3.0, 1.0), (0, 0, 0), 50.0, W, H)
+    a = _allmap(W, H, 5).to(DEV)
+    g = a.clone().requires_grad_(True)
+    assert surface_maps(cam, g)["rend_normal"].requires_grad
+    with torch.no_grad():
+        ref = surface_maps(cam, g)
+    out = surface_maps(cam, a.permute(0, 2, 1).contiguous().permute(0, 2, 1))
+    for k in ("surf_depth", "rend_normal"):
+        np.testing.assert_allclose(out[k].cpu().numpy(), ref[k].cpu().numpy(), atol=1e-6)
