@@ -1547,52 +1547,95 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(const Preproce
   dm2[1] = (float)((double)(dTm[5] * depth) * 0.5 * (double)(float)p.H);
 }
 
-// kernel_grid_backward + kernel_input_backward (gridencoder.cu:245-366) with
-// the dy_dx of kernel_grid (:196-242), D = 3, binary32 tables: one lane per
-// point, levels in order, table gradients as float atomics, the input
-// gradient summed level by level and written once.
+// Cell, weights and corner indices of point u at level l, the interpolation's
+// weights and their derivatives included.
+template <int F>
+__device__ __forceinline__ void encode_corners(const GridEncodeBwdParams& p, int l, const float u[3], float pos[3],
+                                               float der[3], uint32_t gc[3], LevelCorners& cn) {
+  const float off = p.align_corners ? 0.0f : 0.5f;
+  const float scale = p.lv.scale[l];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const float x = u[d] * scale + off;
+    gc[d] = f2u_sat(x);
+    pos[d] = x - (float)gc[d];
+    if (p.interp == 1) {
+      der[d] = 6.0f * pos[d] * (1.0f - pos[d]);
+      pos[d] = pos[d] * pos[d] * (3.0f - 2.0f * pos[d]);
+    } else {
+      der[d] = 1.0f;
+    }
+  }
+  level_corners<F, false>(p.lv, l, off, 0u, u, cn);
+  cn.wx[0] = 1 - pos[0]; cn.wx[1] = pos[0];
+  cn.wy[0] = 1 - pos[1]; cn.wy[1] = pos[1];
+  cn.wz[0] = 1 - pos[2]; cn.wz[1] = pos[2];
+}
+
+__device__ __forceinline__ bool encode_outside(const float u[3]) {
+  return u[0] < 0 || u[0] > 1 || u[1] < 0 || u[1] > 1 || u[2] < 0 || u[2] > 1;
+}
+
+// kernel_grid_backward (gridencoder.cu:245-313), D = 3, binary32 tables: one
+// wave per 64 points and level, through the render backward's scatter.  The
+// bound is the memory side's rate of atomic requests, 20.9 G/s of (instruction,
+// 64-byte segment) whatever the address: an atomic per lane, corner and
+// feature was 8F requests per point and level; the scatter's instructions
+// carry whole x-pairs of entries, ~4.5 requests per cell, and points of one
+// cell are summed first.  142,648 random points on 16 levels of 2^19 entries,
+// F = 2: 2218 -> 660 us (490 at that rate); 2,000,000 points in image order: 82 -> 2.1 ms.  Levels over the grid's y: a wave's scatter is
+// a serial chain, and 142,648 points alone are two waves per SIMD.
 template <int F>
 __global__ void __launch_bounds__(256) grid_encode_backward_kernel(const GridEncodeBwdParams p) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= p.B) return;
-  const float u[3] = {p.inputs[3 * b], p.inputs[3 * b + 1], p.inputs[3 * b + 2]};
-  const bool oob = u[0] < 0 || u[0] > 1 || u[1] < 0 || u[1] > 1 || u[2] < 0 || u[2] > 1;
-  float gi[3] = {0.0f, 0.0f, 0.0f};
-  if (!oob) {
-    const nest_i32x4 rsrc = table_rsrc_rows<F, false>(p.table, p.table_rows);
-    const float off = p.align_corners ? 0.0f : 0.5f;
-    for (int l = 0; l < p.L; l++) {
-      const float scale = p.lv.scale[l];
-      float pos[3], der[3];
+  __shared__ uint32_t stage[4][256];
+  const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int l = (int)blockIdx.y;
+  const uint32_t wid = threadIdx.x >> 6;
+  float cv[8 * F];
 #pragma unroll
-      for (int d = 0; d < 3; d++) {
-        const float x = u[d] * scale + off;
-        pos[d] = x - (float)f2u_sat(x);
-        if (p.interp == 1) {
-          der[d] = 6.0f * pos[d] * (1.0f - pos[d]);
-          pos[d] = pos[d] * pos[d] * (3.0f - 2.0f * pos[d]);
-        } else {
-          der[d] = 1.0f;
-        }
-      }
-      LevelCorners cn;
-      level_corners<F, false>(p.lv, l, off, 0u, u, cn);
-      cn.wx[0] = 1 - pos[0]; cn.wx[1] = pos[0];
-      cn.wy[0] = 1 - pos[1]; cn.wy[1] = pos[1];
-      cn.wz[0] = 1 - pos[2]; cn.wz[1] = pos[2];
-      float gr[F];
+  for (int i = 0; i < 8 * F; i++) cv[i] = 0.0f;
+  uint32_t gc[3] = {0u, 0u, 0u};
+  LevelCorners cn;
+#pragma unroll
+  for (int k = 0; k < 8; k++) cn.idx[k] = 0u;
+  bool on = false;
+  if (b < p.B) {
+    const float u[3] = {p.inputs[3 * b], p.inputs[3 * b + 1], p.inputs[3 * b + 2]};
+    on = !encode_outside(u);
+    if (on) {
+      float pos[3], der[3], gr[F];
+      encode_corners<F>(p, l, u, pos, der, gc, cn);
 #pragma unroll
       for (int f = 0; f < F; f++) gr[f] = p.grad[(size_t)b * p.L * F + (size_t)l * F + f];
-      float* dl = p.grad_table + (size_t)p.lv.base[l] * F;
 #pragma unroll
       for (int k = 0; k < 8; k++) {
         const float wk = (1.0f * cn.wx[k & 1]) * cn.wy[(k >> 1) & 1] * cn.wz[k >> 2];
 #pragma unroll
-        for (int f = 0; f < F; f++) atomic_add(dl + (size_t)cn.idx[k] * F + f, wk * gr[f]);
+        for (int f = 0; f < F; f++) cv[k * F + f] = wk * gr[f];
       }
-      if (!p.grad_inputs) continue;
-      float vals[8][F];
+    }
+  }
+  scatter_level<F>(on, gc, cn.idx, cv, p.grad_table + (size_t)p.lv.base[l] * F, stage[wid]);
+}
+
+// kernel_input_backward (gridencoder.cu:316-366) with the dy_dx of kernel_grid
+// (:196-242): one lane per point, summed level by level and written once.
+template <int F>
+__global__ void __launch_bounds__(256) grid_encode_input_backward_kernel(const GridEncodeBwdParams p) {
+  const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (b >= p.B) return;
+  const float u[3] = {p.inputs[3 * b], p.inputs[3 * b + 1], p.inputs[3 * b + 2]};
+  float gi[3] = {0.0f, 0.0f, 0.0f};
+  if (!encode_outside(u)) {
+    const nest_i32x4 rsrc = table_rsrc_rows<F, false>(p.table, p.table_rows);
+    for (int l = 0; l < p.L; l++) {
+      float pos[3], der[3], gr[F], vals[8][F];
+      uint32_t gc[3];
+      LevelCorners cn;
+      encode_corners<F>(p, l, u, pos, der, gc, cn);
       corners_load<F, false>(rsrc, cn, vals);
+#pragma unroll
+      for (int f = 0; f < F; f++) gr[f] = p.grad[(size_t)b * p.L * F + (size_t)l * F + f];
 #pragma unroll
       for (int gd = 0; gd < 3; gd++) {
         float rg[F];
@@ -1600,7 +1643,7 @@ __global__ void __launch_bounds__(256) grid_encode_backward_kernel(const GridEnc
         for (int f = 0; f < F; f++) rg[f] = 0.0f;
 #pragma unroll
         for (int idx = 0; idx < 4; idx++) {
-          float wgt = scale;
+          float wgt = p.lv.scale[l];
           int kl = 0;
 #pragma unroll
           for (int nd = 0; nd < 2; nd++) {
@@ -1618,25 +1661,29 @@ __global__ void __launch_bounds__(256) grid_encode_backward_kernel(const GridEnc
       }
     }
   }
-  if (p.grad_inputs) {
 #pragma unroll
-    for (int d = 0; d < 3; d++) p.grad_inputs[3 * b + d] = gi[d];
-  }
+  for (int d = 0; d < 3; d++) p.grad_inputs[3 * b + d] = gi[d];
+}
+
+template <int F>
+hipError_t launch_encode_bwd(const GridEncodeBwdParams& p, hipStream_t s) {
+  const unsigned blocks = (unsigned)((p.B + 255) / 256);
+  hipLaunchKernelGGL(grid_encode_backward_kernel<F>, dim3(blocks, (unsigned)p.L), dim3(256), 0, s, p);
+  if (p.grad_inputs) hipLaunchKernelGGL(grid_encode_input_backward_kernel<F>, dim3(blocks), dim3(256), 0, s, p);
+  return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_grid_encode_backward(const GridEncodeBwdParams& p, hipStream_t s) {
   if (p.B == 0) return hipSuccess;
-  const dim3 grid((unsigned)((p.B + 255) / 256));
   switch (p.F) {
-    case 1: hipLaunchKernelGGL(grid_encode_backward_kernel<1>, grid, dim3(256), 0, s, p); break;
-    case 2: hipLaunchKernelGGL(grid_encode_backward_kernel<2>, grid, dim3(256), 0, s, p); break;
-    case 4: hipLaunchKernelGGL(grid_encode_backward_kernel<4>, grid, dim3(256), 0, s, p); break;
-    case 8: hipLaunchKernelGGL(grid_encode_backward_kernel<8>, grid, dim3(256), 0, s, p); break;
+    case 1: return launch_encode_bwd<1>(p, s);
+    case 2: return launch_encode_bwd<2>(p, s);
+    case 4: return launch_encode_bwd<4>(p, s);
+    case 8: return launch_encode_bwd<8>(p, s);
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 // Workgroups per tile of the grid path, each with every parts-th level: few

@@ -229,6 +229,27 @@ def test_grid_encode_backward_parity(oracle, interp, align):
     assert oob.any() and not xt.grad.cpu().numpy()[oob].any()
 
 
+@pytest.mark.parametrize("F", [1, 2, 4, 8])
+@pytest.mark.parametrize("B,spread", [(1, 1.0), (63, 0.02), (257, 1.0), (4133, 0.0), (4133, 0.05), (20000, 1.0)])
+def test_grid_encode_backward_cells(oracle, F, B, spread):
+    """Ragged point counts, and points spread over the grid, crowded into few
+    cells (the sums of many lanes) or all equal (one cell a level), with some
+    outside: 8 * B binary32 adds in any order onto an entry at most."""
+    from gridencoder import GridEncoder
+    rng = np.random.default_rng(B + F)
+    enc = GridEncoder(3, 6, F, 1.6, 16, 13).to(DEV)
+    x = (0.4 + spread * rng.uniform(-0.41, 0.61, (B, 3))).astype(np.float32)
+    xt = _t(x).requires_grad_(True)
+    y = enc(xt)
+    g = rng.standard_normal(tuple(y.shape)).astype(np.float32)
+    y.backward(_t(g))
+    tab = enc.embeddings.detach().cpu().numpy()
+    grid = oracle.make_grid(6, F, float(np.log2(1.6)), 16, enc._offsets_host, tab, (0.0, 1.0), False)
+    gt, gi = oracle.grid_encode_backward(grid, x, g)
+    assert _rel(enc.embeddings.grad.cpu().numpy(), gt) < TOL
+    assert _rel(xt.grad.cpu().numpy(), gi) < TOL
+
+
 def test_autograd_through_drop_in_rasterizer():
     """GaussianRasterizer forward + loss.backward() (the reference's training
     call, DSRpy:174-275) lands the same gradients in .grad as a direct
