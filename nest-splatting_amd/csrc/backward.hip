@@ -103,6 +103,19 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 __device__ __forceinline__ void atomic_add(float* p, float v) { unsafeAtomicAdd(p, v); }
 
+__device__ __forceinline__ void lds_add(float* a, float v) {
+  __hip_atomic_fetch_add(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Between LDS accesses of different lanes of one wave (which the hardware
+// keeps in order): the compiler moves no memory access across it, whatever
+// the types the accesses are made with.
+__device__ __forceinline__ void wave_lds_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // Staging area of the table-gradient atomics: 256 dwords of LDS per wave,
 // kSlots slots of NV = 8F summed values (a cell's corner values, corner-major)
 // followed by the slots' 8 entry indices.  A flush adds nb slots with packed
@@ -121,6 +134,7 @@ __device__ __forceinline__ void stage_flush(const uint32_t* st, uint32_t nb, flo
   constexpr uint32_t kIdx = StageLayout<F>::kIdx;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t nval = nb * NV;
+  wave_lds_order();
   for (uint32_t f0 = 0; f0 < nval; f0 += 64u) {
     const uint32_t f = f0 + lane;
     if (f < nval) {
@@ -130,125 +144,134 @@ __device__ __forceinline__ void stage_flush(const uint32_t* st, uint32_t nb, flo
       if (val != 0.0f) atomic_add(dl + (size_t)e * F + (v % F), val);
     }
   }
+  wave_lds_order();
 }
 
-constexpr uint32_t kSmallCell = 8;  // cells of up to this many lanes are summed by pointer jumping
+constexpr int kScatterAux = 128;   // dwords of LDS per wave beside the staging area
+constexpr uint32_t kFewCells = 8;  // mean lanes per cell above which cells are summed in registers
 
 // Table gradient of one level for the wave (uniform control flow): lanes
 // whose hits fall in the same cell (same g) share all eight corner entries.
-// The cells are taken one at a time (the lowest remaining lane's cell and
-// every lane sharing it).  A cell of more than kSmallCell lanes has its 8F
-// values summed over its lanes with recursive-halving reduce-scatters, 16
-// values at a time (after one, lane l holds the sum of value l / 4 of the
-// chunk), written straight to a staging slot; the smaller cells are summed all
-// at once after the search by pointer jumping along each cell's lanes, into
-// the cell's lowest lane, which then writes a slot as a lane alone in its cell
-// does.  Full sets of slots are added with packed atomics.  At coarse levels a wave's 64 hits
-// (neighbouring pixels and splats adjacent in depth) are a few cells, which is
-// where the per-lane atomics of the reference pile onto the same addresses; at
-// fine levels a cell holds a few lanes.
+// Every lane writes its number into a 512-byte table in LDS at a hash of its
+// cell; the lane that is left there, if its cell is the same, leads the lane's
+// cell (a lane that finds another cell there goes alone, which costs its
+// merging and nothing else).
+//  - Few cells (coarse levels: neighbouring pixels and splats adjacent in
+//    depth): a cell's 8F values are summed over its lanes with
+//    recursive-halving reduce-scatters, 16 values at a time (after one, lane l
+//    holds the sum of value l / 4 of the chunk), written straight to a staging
+//    slot; full sets of slots are added with packed atomics.
+//  - Otherwise the cells are numbered, and one x-pair of corners at a time the
+//    leaders write their 2F values to their cell's slot, the other lanes add
+//    theirs there (LDS atomics) and the slots are added to memory, consecutive
+//    values by consecutive lanes, so that an x-pair of entries is one request
+//    where it lies in one 64-byte segment.
+// Finding the cells one at a time by ballots and summing the small ones by
+// pointer jumping took SCAT_OLD ms of the backward of an 801x517 frame of 16
+// levels, where this takes SCAT_NEW.
 template <int F>
-__device__ __forceinline__ void scatter_level(bool on, const uint32_t gc[3], const uint32_t idx[8], float* cv,
-                                              float* dl, uint32_t* st) {
+__device__ __forceinline__ void scatter_level(bool on, const uint32_t gc[3], const uint32_t idx[8], const float* cv,
+                                              float* dl, uint32_t* st, uint32_t* aux) {
   constexpr int NV = 8 * F;
   constexpr uint32_t kSlots = StageLayout<F>::kSlots;
   constexpr uint32_t kIdx = StageLayout<F>::kIdx;
   const uint32_t lane = threadIdx.x & 63u;
-  uint64_t rem = __ballot(on);
-  uint64_t issue = 0ull;  // lanes holding a small cell's sum (or alone in their cell)
-  // next lane of the lane's small cell as a byte address for ds_bpermute;
-  // bit 31 set: the lane is the last of its cell (or in no small cell)
-  uint32_t succ = 0x80000000u | (lane << 2);
-  uint32_t small_max = 1u;
-  uint32_t nb = 0u;  // staging slots in use
-  while (rem != 0ull) {
-    const int ld = __ffsll((long long)rem) - 1;
-    const uint32_t k0 = __builtin_amdgcn_readlane(gc[0], ld), k1 = __builtin_amdgcn_readlane(gc[1], ld),
-                   k2 = __builtin_amdgcn_readlane(gc[2], ld);
-    const uint64_t m = __ballot(gc[0] == k0) & __ballot(gc[1] == k1) & __ballot(gc[2] == k2) & rem;
-    rem &= ~m;
-    const uint32_t n = (uint32_t)__popcll(m);
-    if (n <= kSmallCell) {
-      issue |= m & (~m + 1ull);
-      if (n > 1u) {
-        const uint64_t after = m & ~((2ull << lane) - 1ull);
-        if (((m >> lane) & 1ull) != 0ull && after != 0ull) succ = (uint32_t)(__ffsll((long long)after) - 1) << 2;
-        small_max = n > small_max ? n : small_max;
+  const uint64_t onm = __ballot(on);
+  if (onm == 0ull) return;
+  wave_lds_order();
+  volatile uint8_t* tab = reinterpret_cast<volatile uint8_t*>(aux);
+  const uint32_t h = ((gc[0] + gc[1] * 2654435761u + gc[2] * 805459861u) * 2246822519u) >> 23;
+  if (on) tab[h] = (uint8_t)lane;
+  wave_lds_order();
+  uint32_t ld = on ? (uint32_t)tab[h] : lane;
+  {
+    const int at = (int)(ld << 2);
+    const bool same = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)gc[0]) == gc[0] &
+                      (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)gc[1]) == gc[1] &
+                      (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)gc[2]) == gc[2];
+    ld = same ? ld : lane;
+  }
+  const bool lead = on && ld == lane;
+  uint64_t leaders = __ballot(lead);
+  const uint32_t cells = (uint32_t)__popcll(leaders);
+  wave_lds_order();
+  if ((uint32_t)__popcll(onm) > cells * kFewCells) {
+    uint32_t nb = 0u;  // staging slots in use
+    while (leaders != 0ull) {
+      const int l0 = __ffsll((long long)leaders) - 1;
+      leaders &= leaders - 1ull;
+      const bool mem = on && ld == (uint32_t)l0;
+      if (nb == kSlots) {
+        stage_flush<F>(st, nb, dl);
+        nb = 0u;
       }
-      continue;
-    }
-    const bool mem = ((m >> lane) & 1ull) != 0ull;
-    if (nb == kSlots) {
-      stage_flush<F>(st, nb, dl);
-      nb = 0u;
-    }
-    // reduce-scatter in chunks of kCh values (fewer live registers)
-    constexpr int kCh = NV < 16 ? NV : 16;
-    constexpr int kRepC = 64 / kCh;
+      // reduce-scatter in chunks of kCh values (fewer live registers)
+      constexpr int kCh = NV < 16 ? NV : 16;
+      constexpr int kRepC = 64 / kCh;
 #pragma unroll
-    for (int c = 0; c < NV / kCh; c++) {
-      float v[kCh];
+      for (int c = 0; c < NV / kCh; c++) {
+        float v[kCh];
 #pragma unroll
-      for (int i = 0; i < kCh; i++) v[i] = mem ? cv[c * kCh + i] : 0.0f;
-      int vi = 0;
+        for (int i = 0; i < kCh; i++) v[i] = mem ? cv[c * kCh + i] : 0.0f;
+        int vi = 0;
 #pragma unroll
-      for (int s = 0; (kCh >> (s + 1)) >= 1; s++) {
-        const int h = kCh >> (s + 1);
-        const int bit = 5 - s;
+        for (int s = 0; (kCh >> (s + 1)) >= 1; s++) {
+          const int hh = kCh >> (s + 1);
+          const int bit = 5 - s;
 #pragma unroll
-        for (int i = 0; i < h; i++) v[i] = halve(bit, v[i], v[i + h]);
-        if (((lane >> bit) & 1u) != 0u) vi += h;
+          for (int i = 0; i < hh; i++) v[i] = halve(bit, v[i], v[i + hh]);
+          if (((lane >> bit) & 1u) != 0u) vi += hh;
+        }
+        // lanes differing only in the bits below hold the same value index
+#pragma unroll
+        for (int bit = 0; (1 << bit) < kRepC; bit++) v[0] = halve(bit, v[0], v[0]);
+        if ((lane % kRepC) == 0u) st[nb * NV + (uint32_t)(c * kCh + vi)] = __float_as_uint(v[0]);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      // lanes differing only in the bits below hold the same value index
+      uint32_t e = __builtin_amdgcn_readlane(idx[0], l0);
 #pragma unroll
-      for (int bit = 0; (1 << bit) < kRepC; bit++) v[0] = halve(bit, v[0], v[0]);
-      if ((lane % kRepC) == 0u) st[nb * NV + (uint32_t)(c * kCh + vi)] = __float_as_uint(v[0]);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int kk = 1; kk < 8; kk++) {
+        const uint32_t ek = __builtin_amdgcn_readlane(idx[kk], l0);
+        e = (lane == (uint32_t)kk) ? ek : e;
+      }
+      if (lane < 8u) st[kIdx + nb * 8u + lane] = e;
+      nb++;
     }
-    uint32_t e = __builtin_amdgcn_readlane(idx[0], ld);
-#pragma unroll
-    for (int kk = 1; kk < 8; kk++) {
-      const uint32_t ek = __builtin_amdgcn_readlane(idx[kk], ld);
-      e = (lane == (uint32_t)kk) ? ek : e;
-    }
-    if (lane < 8u) st[kIdx + nb * 8u + lane] = e;
-    nb++;
+    stage_flush<F>(st, nb, dl);
+    wave_lds_order();
+    return;
   }
-  // small cells: pointer jumping, after which a cell's lowest lane holds the
-  // sum over the cell's lanes
-  for (uint32_t span = 1u; span < small_max; span <<= 1) {
-    const bool has = (succ & 0x80000000u) == 0u;
-    const int addr = (int)(succ & 0xFFu);
+  constexpr uint32_t kPair = 2 * F;                                   // values of an x-pair of corners
+  constexpr uint32_t kCells = 256u / kPair < 64u ? 256u / kPair : 64u;  // cells whose pairs fit the staging area
+  const uint32_t rank = (uint32_t)__popcll(leaders & ((1ull << lane) - 1ull));
+  const uint32_t cell = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(ld << 2), (int)rank);
+  float* sums = reinterpret_cast<float*>(st);
+  for (uint32_t c0 = 0; c0 < cells; c0 += kCells) {
+    const uint32_t slot = cell - c0;  // past kCells for the cells before c0
+    const bool in = on && slot < kCells;
+    const uint32_t nval = min(kCells, cells - c0) * kPair;
 #pragma unroll
-    for (int i = 0; i < NV; i++) {
-      const float got = __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(cv[i])));
-      if (has) cv[i] += got;
-      if ((i & 7) == 7) __builtin_amdgcn_sched_barrier(0);
-    }
-    if (span * 2u < small_max) succ = (uint32_t)__builtin_amdgcn_ds_bpermute(addr, (int)succ);
-  }
-  const uint32_t n_iss = (uint32_t)__popcll(issue);
-  const uint32_t rank = (uint32_t)__popcll(issue & ((1ull << lane) - 1ull));
-  const bool me = ((issue >> lane) & 1ull) != 0ull;
-  for (uint32_t done = 0; done < n_iss;) {
-    if (nb == kSlots) {
-      stage_flush<F>(st, nb, dl);
-      nb = 0u;
-    }
-    const uint32_t take = min(kSlots - nb, n_iss - done);
-    if (me && rank >= done && rank < done + take) {
-      const uint32_t h = nb + rank - done;
-      float4* sv = reinterpret_cast<float4*>(st + h * NV);
+    for (int c = 0; c < 4; c++) {
+      if (in && lead) {
 #pragma unroll
-      for (int i = 0; i < NV / 4; i++) sv[i] = make_float4(cv[4 * i], cv[4 * i + 1], cv[4 * i + 2], cv[4 * i + 3]);
-      uint4* si = reinterpret_cast<uint4*>(st + kIdx + h * 8u);
-      si[0] = make_uint4(idx[0], idx[1], idx[2], idx[3]);
-      si[1] = make_uint4(idx[4], idx[5], idx[6], idx[7]);
+        for (uint32_t i = 0; i < kPair; i += 2)
+          *reinterpret_cast<float2*>(sums + slot * kPair + i) = make_float2(cv[c * kPair + i], cv[c * kPair + i + 1]);
+        *reinterpret_cast<uint2*>(aux + 2u * slot) = make_uint2(idx[2 * c], idx[2 * c + 1]);
+      }
+      wave_lds_order();
+      if (in && !lead) {
+#pragma unroll
+        for (uint32_t i = 0; i < kPair; i++) lds_add(sums + slot * kPair + i, cv[c * kPair + i]);
+      }
+      wave_lds_order();
+      for (uint32_t f = lane; f < nval; f += 64u) {
+        const float val = sums[f];
+        const uint32_t e = aux[f / F];
+        if (val != 0.0f) atomic_add(dl + (size_t)e * F + (f % F), val);
+      }
+      wave_lds_order();
     }
-    nb += take;
-    done += take;
   }
-  if (nb > 0u) stage_flush<F>(st, nb, dl);
 }
 
 // query_feature<true> for the wave's hits at grid coordinates u (lanes with
@@ -259,7 +282,7 @@ __device__ __forceinline__ void scatter_level(bool on, const uint32_t gc[3], con
 template <int F>
 __device__ __forceinline__ void hash_backward_wave(const GridParams& g, nest_i32x4 rsrc, const float u[3],
                                                    float grad_scale, uint32_t lane_levels, float w,
-                                                   const float* dpix, size_t HW, float* dtable, uint32_t* st,
+                                                   const float* dpix, size_t HW, float* dtable, uint32_t* st, uint32_t* aux,
                                                    uint32_t first, uint32_t step, float& dot, float dxyz[3]) {
   dot = 0.0f;
   dxyz[0] = dxyz[1] = dxyz[2] = 0.0f;
@@ -338,7 +361,7 @@ __device__ __forceinline__ void hash_backward_wave(const GridParams& g, nest_i32
         for (int f = 0; f < F; f++) dxyz[gd] += gf[f] * rg[f];
       }
     }
-    scatter_level<F>(on, gc, cn.idx, cv, dtable + (size_t)lv.base[l] * F, st);
+    scatter_level<F>(on, gc, cn.idx, cv, dtable + (size_t)lv.base[l] * F, st, aux);
   }
 }
 
@@ -650,9 +673,6 @@ constexpr uint32_t kSumT = 0, kSumM = 9, kSumN = 11, kSumO = 14, kSumK = 15;
 constexpr uint32_t kSumCol = 16, kSumColour = 19;             // colour path: 3 colours
 constexpr uint32_t kSumH = 16, kSumS = 25, kSumW = 26, kSumHash = 27;  // grid path
 
-__device__ __forceinline__ void lds_add(float* a, float v) {
-  __hip_atomic_fetch_add(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
 
 constexpr uint32_t kBigGroup = 8;   // lanes at one splat that are summed in registers first
 
@@ -1113,6 +1133,7 @@ render_backward_kernel(const RenderBwdParams p) {
   __shared__ uint64_t lact[kBwdWaves][kBwdWide];      // the segment's first splats: lanes hit, batch index
   __shared__ uint8_t lj[kBwdWaves][kBwdWide];
   __shared__ uint64_t smask[kBwdWaves][kMasks];
+  __shared__ __attribute__((aligned(8))) uint32_t saux[kBwdWaves][kScatterAux];
 
   // level parts: workgroup b runs on XCD b % 8, dealt as in the forward
   uint32_t pos = blockIdx.x, part = 0u;
@@ -1232,7 +1253,7 @@ render_backward_kernel(const RenderBwdParams p) {
         // the chunk's queue entries (read above, rewritten below) stage the
         // table-gradient atomics meanwhile
         hash_backward_wave<F>(g, rsrc, u, gsc, lev, w, dp, HW, p.dtable, reinterpret_cast<uint32_t*>(&hq[wid][r0]),
-                              part, p.parts, dot, dxyz);
+                              saux[wid], part, p.parts, dot, dxyz);
         if (on) hq[wid][e] = make_float4(dot, dxyz[0], dxyz[1], dxyz[2]);
       }
       __builtin_amdgcn_wave_barrier();
@@ -1587,7 +1608,8 @@ __device__ __forceinline__ bool encode_outside(const float u[3]) {
 // a serial chain, and 142,648 points alone are two waves per SIMD.
 template <int F>
 __global__ void __launch_bounds__(256) grid_encode_backward_kernel(const GridEncodeBwdParams p) {
-  __shared__ uint32_t stage[4][256];
+  __shared__ __attribute__((aligned(16))) uint32_t stage[4][256];
+  __shared__ __attribute__((aligned(8))) uint32_t saux[4][kScatterAux];
   const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int l = (int)blockIdx.y;
   const uint32_t wid = threadIdx.x >> 6;
@@ -1615,7 +1637,7 @@ __global__ void __launch_bounds__(256) grid_encode_backward_kernel(const GridEnc
       }
     }
   }
-  scatter_level<F>(on, gc, cn.idx, cv, p.grad_table + (size_t)p.lv.base[l] * F, stage[wid]);
+  scatter_level<F>(on, gc, cn.idx, cv, p.grad_table + (size_t)p.lv.base[l] * F, stage[wid], saux[wid]);
 }
 
 // kernel_input_backward (gridencoder.cu:316-366) with the dy_dx of kernel_grid
