@@ -1198,11 +1198,14 @@ int nest_backward(const nest_raster_settings* rs, const nest_hashgrid* gr, const
                {io->dL_drotations, (int64_t)P * 4}, {from_sh ? io->dL_dshs : nullptr, (int64_t)P * M * 3},
                {hash ? io->dL_dfeatures : nullptr, hash ? (int64_t)gr->table_rows * gr->level_dim : 0},
                {io->dL_dshapes, (int64_t)P}};
+  FillList zero{};
+  static_assert(sizeof(fills) / sizeof(fills[0]) <= kFillMax, "one launch");
   for (const Fill& f : fills) {
-    if (!f.p || f.n == 0) continue;
-    hipError_t e = launch_fill_u32(reinterpret_cast<uint32_t*>(f.p), 0u, f.n, s);
-    if (e != hipSuccess) return hip_fail(e, "backward fill");
+    zero.dst[zero.count] = reinterpret_cast<uint32_t*>(f.p);
+    zero.n[zero.count++] = f.n;
   }
+  hipError_t ez = launch_fill_list(zero, 0u, s);
+  if (ez != hipSuccess) return hip_fail(ez, "backward fill");
   if (P == 0) return NEST_OK;
 
   RenderBwdParams rp{};

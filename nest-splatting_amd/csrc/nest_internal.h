@@ -209,6 +209,15 @@ hipError_t launch_centre_rgb(const GridParams& g, int P, const float* homotrans,
 // plus the grid p.grid at its blended position (out_others 8-10) with the
 // appearance level of the tile's first splat (0 without hits or ap_level).
 hipError_t launch_spatial_add(const RenderParams& p, const float* ap_level, hipStream_t s);
+// Arrays of 32-bit words filled in one launch (null or empty ones skipped).
+constexpr int kFillMax = 16;
+struct FillList {
+  int count;
+  uint32_t* dst[kFillMax];
+  int64_t n[kFillMax];
+  uint32_t first[kFillMax];  // set by launch_fill_list
+};
+hipError_t launch_fill_list(FillList list, uint32_t value, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* dst, uint32_t value, int64_t n, hipStream_t s);
 
 // Backward of the render (renderCUDAsurfelBackward, mode 0).  Reads the

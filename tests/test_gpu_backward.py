@@ -250,6 +250,24 @@ def test_grid_encode_backward_cells(oracle, F, B, spread):
     assert _rel(xt.grad.cpu().numpy(), gi) < TOL
 
 
+@pytest.mark.parametrize("rows", [4920, 4921, 8193, 40003])
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+def test_gradient_zeroed_at_any_alignment(rows, shift):
+    """The table gradient's fill (16-byte stores between an array's first and
+    last 16-byte boundary) touches its array and nothing beside it."""
+    import ctypes as ct
+
+    from nest_splat import _lib as L
+    buf = torch.ones((rows + 16,), device=DEV)
+    offs = (ct.c_int32 * 2)(0, 4920)
+    L.check(L.lib().nest_grid_encode_backward(None, 0, 3, None, rows, L.DTYPE_F32, offs, 1, 1, 0.0, 16, 0, 0, 0, None,
+                                              ct.c_void_p(buf.data_ptr() + 4 * (4 + shift)), None, L.stream_ptr(DEV)),
+            "nest_grid_encode_backward")
+    got = buf.cpu().numpy()
+    assert not got[4 + shift: 4 + shift + rows].any()
+    assert (got[:4 + shift] == 1).all() and (got[4 + shift + rows:] == 1).all()
+
+
 def test_autograd_through_drop_in_rasterizer():
     """GaussianRasterizer forward + loss.backward() (the reference's training
     call, DSRpy:174-275) lands the same gradients in .grad as a direct
