@@ -1118,7 +1118,7 @@ __device__ __forceinline__ void bwd_row_grads(const RenderBwdParams& p, bool on,
   }
 }
 
-// Three workgroups per CU (51.8 KB of LDS each) where the registers allow:
+// Three workgroups per CU (52.6 KB of LDS each) where the registers allow:
 // F <= 4 fits 168 VGPRs, F = 8 keeps two.
 template <int F, int kRows>
 __global__ void __launch_bounds__(kBwdThreads) __attribute__((amdgpu_waves_per_eu(F <= 4 ? 3 : 2)))
@@ -1604,8 +1604,9 @@ __device__ __forceinline__ bool encode_outside(const float u[3]) {
 // feature was 8F requests per point and level; the scatter's instructions
 // carry whole x-pairs of entries, ~4.5 requests per cell, and points of one
 // cell are summed first.  142,648 random points on 16 levels of 2^19 entries,
-// F = 2: 2218 -> 660 us (490 at that rate); 2,000,000 points in image order: 82 -> 2.1 ms.  Levels over the grid's y: a wave's scatter is
-// a serial chain, and 142,648 points alone are two waves per SIMD.
+// F = 2: 2218 -> 660 us (490 at that rate); a step of 2,000,000 points in image
+// order: 82 -> 2.1 ms.  Levels over the grid's y: a wave's scatter is a serial
+// chain, and 142,648 points alone are two waves per SIMD.
 template <int F>
 __global__ void __launch_bounds__(256) grid_encode_backward_kernel(const GridEncodeBwdParams p) {
   __shared__ __attribute__((aligned(16))) uint32_t stage[4][256];
