@@ -458,8 +458,6 @@ def _plain_map(t: torch.Tensor) -> bool:
 def _surface_maps_fused(cam, allmap: torch.Tensor, depth_ratio: float) -> dict:
     """surface_maps in one kernel (nest_surface_maps)."""
     H, W = int(allmap.shape[1]), int(allmap.shape[2])
-    if (H, W) != (cam.image_height, cam.image_width):
-        raise ValueError(f"allmap is {H} x {W}, the camera {cam.image_height} x {cam.image_width}")
     normals = torch.empty((2, H, W, 3), dtype=torch.float32, device=allmap.device)
     depths = torch.empty((3, 1, H, W), dtype=torch.float32, device=allmap.device)
     wv = cam.world_view_transform
@@ -481,7 +479,8 @@ def surface_maps(cam, allmap: torch.Tensor, depth_ratio: float = 0.0) -> dict:
     world-space normal map, median and expected depth, distortion, the
     pseudo-surface depth (depth_ratio blends expected and median depth) and
     its normal from the back-projected depth map, scaled by alpha."""
-    if _plain_map(allmap) and type(depth_ratio) in (int, float):
+    if (_plain_map(allmap) and type(depth_ratio) in (int, float) and
+            tuple(allmap.shape[1:]) == (cam.image_height, cam.image_width)):
         return _surface_maps_fused(cam, allmap, depth_ratio)
     dev = allmap.device
     render_alpha = allmap[1:2]

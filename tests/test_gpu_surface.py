@@ -67,3 +67,21 @@ def test_surface_maps_gradient_and_views_keep_the_general_path():
     out = surface_maps(cam, a.permute(0, 2, 1).contiguous().permute(0, 2, 1))
     for k in ("surf_depth", "rend_normal"):
         np.testing.assert_allclose(out[k].cpu().numpy(), ref[k].cpu().numpy(), atol=1e-6)
+
+
+def test_surface_maps_of_another_camera_size_keep_the_general_path():
+    """A map that is not the camera's size does what the tensor operations do
+    with it: broadcast where they broadcast, raise where they raise."""
+    from nest_splat.camera import look_at
+    from nest_splat.renderer import surface_maps
+    cam = look_at((0.4, -3.0, 1.0), (0, 0, 0), 50.0, 1, 9)
+    a = _allmap(9, 1, 3)
+    ref, out = surface_maps(cam, a), surface_maps(cam, a.to(DEV))
+    for k, v in ref.items():
+        assert out[k].shape == v.shape, k
+    np.testing.assert_array_equal(out["surf_depth"].cpu().numpy(), ref["surf_depth"].numpy())
+    cam = look_at((0.4, -3.0, 1.0), (0, 0, 0), 50.0, 24, 10)
+    for H, W in ((20, 12), (5, 7)):
+        for dev in ("cpu", DEV):
+            with pytest.raises(RuntimeError):
+                surface_maps(cam, _allmap(W, H, 4).to(dev))
