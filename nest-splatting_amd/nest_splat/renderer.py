@@ -443,6 +443,18 @@ def _render_hybrid(cam, pc, pipe, bg_color, scaling_modifier, ingp, beta, max_in
     return rets
 
 
+def _ops_followed() -> bool:
+    """Whether a trace, transform or mode may follow tensor operations.  torch
+    has no public names for some of these; without them the answer is yes."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return True
+    try:
+        return (torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None or
+                torch._C._len_torch_dispatch_stack() > 0 or torch._C._is_torch_function_mode_enabled())
+    except AttributeError:
+        return True
+
+
 def _plain_map(t: torch.Tensor) -> bool:
     """Whether a map can go to a kernel as memory: an ordinary contiguous
     float32 device tensor that no gradient, transform, mode or trace follows."""
@@ -450,9 +462,7 @@ def _plain_map(t: torch.Tensor) -> bool:
         return False
     if t.ndim != 3 or t.shape[0] < 8 or t.shape[1] * t.shape[2] >= 1 << 31 or (torch.is_grad_enabled() and t.requires_grad):
         return False
-    return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None and
-            torch._C._len_torch_dispatch_stack() == 0 and not torch._C._is_torch_function_mode_enabled() and
-            not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+    return not _ops_followed()
 
 
 def _surface_maps_fused(cam, allmap: torch.Tensor, depth_ratio: float) -> dict:

@@ -68,3 +68,41 @@ def test_eval_sh_matches_the_oracle(oracle, deg):
     vis = pre["radii"] > 0
     assert vis.sum() > 100
     assert np.abs(mine[vis] - ref[vis]).max() < 2e-6
+
+
+@pytest.mark.parametrize("name", ["autograd.forward_ad._current_level", "_C._functorch.peek_interpreter_stack",
+                                  "_C._len_torch_dispatch_stack", "_C._is_torch_function_mode_enabled"])
+def test_surface_rule_without_a_private_torch_name(monkeypatch, name):
+    """A torch without one of the private names that tell whether a transform
+    or mode is active: the rule says that one may be (the tensor operations),
+    and does not raise."""
+    from nest_splat import renderer
+    assert renderer._ops_followed() is False
+    owner = torch
+    *path, last = name.split(".")
+    for part in path:
+        owner = getattr(owner, part)
+    monkeypatch.delattr(owner, last)
+    followed = renderer._ops_followed()
+    monkeypatch.undo()
+    assert followed is True
+
+
+def test_surface_rule_sees_transforms_and_modes():
+    """Under each of these the surface maps take the tensor operations."""
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from nest_splat import renderer
+    seen = []
+    with forward_ad.dual_level():
+        seen.append(renderer._ops_followed())
+    torch.func.vmap(lambda x: (seen.append(renderer._ops_followed()), x)[1])(torch.zeros(2))
+    with TorchFunctionMode():
+        seen.append(renderer._ops_followed())
+    with TorchDispatchMode():
+        seen.append(renderer._ops_followed())
+    torch.jit.trace(lambda x: (seen.append(renderer._ops_followed()), x + 1)[1], torch.zeros(2), check_trace=False)
+    assert seen == [True] * 5
+    assert renderer._ops_followed() is False
