@@ -468,8 +468,9 @@ def _plain_map(t: torch.Tensor) -> bool:
 def _surface_maps_fused(cam, allmap: torch.Tensor, depth_ratio: float) -> dict:
     """surface_maps in one kernel (nest_surface_maps)."""
     H, W = int(allmap.shape[1]), int(allmap.shape[2])
-    normals = torch.empty((2, H, W, 3), dtype=torch.float32, device=allmap.device)
-    depths = torch.empty((3, 1, H, W), dtype=torch.float32, device=allmap.device)
+    # each map in memory of its own: changed, saved and freed by itself
+    normal, surf_normal = (torch.empty((H, W, 3), dtype=torch.float32, device=allmap.device) for _ in range(2))
+    depth, expected, median = (torch.empty((1, H, W), dtype=torch.float32, device=allmap.device) for _ in range(3))
     wv = cam.world_view_transform
     wv = wv.detach().cpu().numpy() if isinstance(wv, torch.Tensor) else np.asarray(wv)
     f9 = ct.c_float * 9
@@ -477,11 +478,11 @@ def _surface_maps_fused(cam, allmap: torch.Tensor, depth_ratio: float) -> dict:
     M = f9(*view_ray_matrix(cam).reshape(-1).tolist())
     origin = (ct.c_float * 3)(*np.linalg.inv(wv.astype(np.float64).T)[:3, 3].tolist())
     L.check(L.lib().nest_surface_maps(W, H, L.ptr(allmap), R, M, origin, 1 - depth_ratio, depth_ratio,
-                                      L.ptr(normals[0]), L.ptr(depths[0]), L.ptr(normals[1]), L.ptr(depths[1]),
-                                      L.ptr(depths[2]), L.stream_ptr(allmap.device)), "nest_surface_maps")
-    return {"rend_alpha": allmap[1:2], "rend_normal": normals[0].permute(2, 0, 1), "rend_dist": allmap[6:7],
-            "surf_depth": depths[0], "surf_normal": normals[1].permute(2, 0, 1), "gaussian_num": allmap[7:8],
-            "depth_expected": depths[1], "depth_median": depths[2]}
+                                      L.ptr(normal), L.ptr(depth), L.ptr(surf_normal), L.ptr(expected),
+                                      L.ptr(median), L.stream_ptr(allmap.device)), "nest_surface_maps")
+    return {"rend_alpha": allmap[1:2], "rend_normal": normal.permute(2, 0, 1), "rend_dist": allmap[6:7],
+            "surf_depth": depth, "surf_normal": surf_normal.permute(2, 0, 1), "gaussian_num": allmap[7:8],
+            "depth_expected": expected, "depth_median": median}
 
 
 def surface_maps(cam, allmap: torch.Tensor, depth_ratio: float = 0.0) -> dict:

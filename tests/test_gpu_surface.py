@@ -85,3 +85,21 @@ def test_surface_maps_of_another_camera_size_keep_the_general_path():
         for dev in ("cpu", DEV):
             with pytest.raises(RuntimeError):
                 surface_maps(cam, _allmap(W, H, 4).to(dev))
+
+
+def test_surface_maps_have_memory_of_their_own():
+    """A map that a loss saved for its backward is not touched by an in-place
+    change of another map, and a map kept alone keeps no other map's memory."""
+    from nest_splat.camera import look_at
+    from nest_splat.renderer import surface_maps
+    W, H = 33, 20
+    cam = look_at((0.4, -3.0, 1.0), (0, 0, 0), 50.0, W, H)
+    out = surface_maps(cam, _allmap(W, H, 6).to(DEV))
+    names = ("rend_normal", "surf_normal", "surf_depth", "depth_expected", "depth_median")
+    for k in names:
+        assert out[k].untyped_storage().nbytes() == 4 * out[k].numel(), k
+    for saved, changed in zip(names, names[1:] + names[:1]):
+        w = torch.ones((), device=DEV, requires_grad=True)
+        loss = (w * out[saved]).sum()
+        out[changed].add_(1.0)
+        loss.backward()
