@@ -457,8 +457,11 @@ def _ops_followed() -> bool:
 
 def _plain_map(t: torch.Tensor) -> bool:
     """Whether a map can go to a kernel as memory: an ordinary contiguous
-    float32 device tensor that no gradient, transform, mode or trace follows."""
+    float32 tensor of the current device (a launch goes to that one) that no
+    gradient, transform, mode or trace follows."""
     if type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.float32 or not t.is_contiguous():
+        return False
+    if t.device.index != torch.cuda.current_device():
         return False
     if t.ndim != 3 or t.shape[0] < 8 or t.shape[1] * t.shape[2] >= 1 << 31 or (torch.is_grad_enabled() and t.requires_grad):
         return False

@@ -103,3 +103,19 @@ def test_surface_maps_have_memory_of_their_own():
         loss = (w * out[saved]).sum()
         out[changed].add_(1.0)
         loss.backward()
+
+
+def test_surface_maps_of_another_device_keep_the_general_path(monkeypatch):
+    """With another device current, a launch would not be this map's device's."""
+    from nest_splat import renderer
+    from nest_splat.camera import look_at
+    W, H = 33, 20
+    cam = look_at((0.4, -3.0, 1.0), (0, 0, 0), 50.0, W, H)
+    a = _allmap(W, H, 7).to(DEV)
+    assert renderer._plain_map(a)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: DEV.index + 1)
+    assert not renderer._plain_map(a)
+    monkeypatch.setattr(renderer, "_surface_maps_fused", None)
+    out = renderer.surface_maps(cam, a)
+    monkeypatch.undo()
+    np.testing.assert_array_equal(out["surf_depth"].cpu().numpy(), renderer.surface_maps(cam, a)["surf_depth"].cpu().numpy())
