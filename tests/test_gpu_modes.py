@@ -403,9 +403,13 @@ def test_cat_mode_backward_parity(oracle, name, hyb, gl, active):
     CPU tests pin against float64 autograd), on the same forward state.  The
     sums run in another order on each side (per wave then atomically on the
     GPU, sequentially in the oracle): 2e-5 of each array's largest entry."""
+    _cat_backward(oracle, scene(name), hyb, gl, active, 2e-5)
+
+
+def _cat_backward(oracle, sc, hyb, gl, active, tol):
     from nest_splat import rasterizer as rz
-    sc = scene(name)
     sp = sc.spec
+    name = sp.name
     F = sp.F
     pgd = hyb * F
     C = (hyb + gl) * F
@@ -457,7 +461,7 @@ def test_cat_mode_backward_parity(oracle, name, hyb, gl, active):
         assert np.abs(r).max() > 0, k
         err = float(np.abs(o.astype(np.float64) - r).max() / np.abs(r).max())
         print(f"{k}: max rel err {err:.2e}", flush=True)
-        assert err < 2e-5, (k, err)
+        assert err < tol, (k, err)
         if k != "dfeatures":
             assert not o[~vis].any(), k
     if 0 < active < gl:  # the levels past the active ones get no gradient
@@ -584,9 +588,13 @@ def test_adaptive_cat_backward_parity(oracle, mode, name, total, hyb, gl, kt):
     table and the geometry, within 2e-5 of each array's largest entry.  Mode
     14 rows include weight-0 splats, whose grid levels are skipped.  Some
     cases use kernel types 1-3, with dL/dshape."""
+    _adaptive_backward(oracle, mode, scene(name), total, hyb, gl, kt, 2e-5)
+
+
+def _adaptive_backward(oracle, mode, sc, total, hyb, gl, kt, tol):
     from nest_splat import rasterizer as rz
-    sc = scene(name)
     sp = sc.spec
+    name = sp.name
     F = sp.F
     tdim = total * F
     cam = sc.cameras[0]
@@ -650,6 +658,36 @@ def test_adaptive_cat_backward_parity(oracle, mode, name, total, hyb, gl, kt):
         assert np.abs(r).max() > 0, k
         err = float(np.abs(o.astype(np.float64) - r).max() / np.abs(r).max())
         print(f"{k}: max rel err {err:.2e}", flush=True)
-        assert err < 2e-5, (k, err)
+        assert err < tol, (k, err)
         if k != "dfeatures":
             assert not o[~vis].any(), k
+
+
+# (render mode, W, H, total levels, per-splat levels, grid levels, F): the
+# backward's level parts with feature rows, on both sides of the rule's lines
+# (320 tiles below 4 levels, 320 and 768 up to 8, 2560 beyond), so that the
+# rows' gradients and products are sent by part 0 of several workgroups and by
+# a tile's only one; and an ordinary frame with one workgroup per tile.  The
+# wide frames' splats cover thousands of pixels (a 50 degree view up to 40,976
+# pixels wide), so a row's entry sums up to W H ~ 2e5 pixels of a few hits, n =
+# 1e6 terms of both signs, where 2e-5 is for a few thousand: a sequential
+# float32 sum errs by about u sqrt(n) = 6e-5 of its largest partial sum, on
+# both sides: 1e-4.
+ROW_EDGE_TOL = 1e-4
+ROW_EDGE_CASES = [(4, 320 * 16, 9, 5, 2, 3, 8), (4, 321 * 16, 9, 8, 5, 3, 4), (4, 768 * 16 - 5, 7, 8, 3, 5, 2),
+                  (4, 769 * 16, 7, 13, 5, 8, 4), (4, 2560 * 16, 5, 12, 2, 10, 2), (4, 2561 * 16, 5, 12, 3, 9, 4),
+                  (4, 401, 399, 6, 3, 3, 4), (12, 320 * 16, 9, 6, 3, 3, 8), (12, 321 * 16, 9, 6, 3, 3, 4),
+                  (12, 768 * 16, 7, 8, 2, 6, 4), (12, 769 * 16 - 3, 7, 7, 3, 4, 8), (12, 2561 * 16, 5, 12, 3, 9, 2),
+                  (12, 401, 399, 6, 3, 3, 4), (14, 321 * 16, 9, 6, 3, 3, 4), (14, 769 * 16, 7, 8, 2, 6, 2),
+                  (14, 401, 399, 8, 5, 3, 8), (7, 769 * 16, 7, 6, 0, 6, 4), (7, 401, 399, 3, 0, 3, 2)]
+
+
+@pytest.mark.parametrize("mode,W,H,total,hyb,gl,F", ROW_EDGE_CASES)
+def test_row_backward_level_parts(oracle, mode, W, H, total, hyb, gl, F):
+    from nest_splat.scene import get_spec, make_scene
+    sc = make_scene(get_spec("cfg2", name=f"rows {W}x{H} F={F}", P=6000, W=W, H=H, L=max(total, gl), F=F, log2T=13,
+                             log_scale_mu=-3.0))
+    if mode == 4:
+        _cat_backward(oracle, sc, hyb, gl, gl, ROW_EDGE_TOL)
+    else:
+        _adaptive_backward(oracle, mode, sc, total, hyb, gl, 0, ROW_EDGE_TOL)
