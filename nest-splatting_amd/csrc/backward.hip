@@ -741,8 +741,9 @@ __device__ __forceinline__ void bwd_row_geometry(const BwdGrad& gr, float* v) {
 
 // Adds n consecutive sums of every staged splat to dst rows of `stride`
 // floats and clears them; consecutive lanes take consecutive floats of a row.
-template <uint32_t kRow, uint32_t n>
-__device__ __forceinline__ void bwd_flush(float* sums, uint32_t first, uint32_t splats, const uint32_t* sid, float* dst,
+// id(j) is the splat staged at j.
+template <uint32_t kRow, uint32_t n, typename Id>
+__device__ __forceinline__ void bwd_flush(float* sums, uint32_t first, uint32_t splats, const Id& id, float* dst,
                                           uint32_t stride) {
   for (uint32_t i = threadIdx.x; i < splats * n; i += kBwdThreads) {
     const uint32_t j = i / n, r = i % n;
@@ -750,19 +751,19 @@ __device__ __forceinline__ void bwd_flush(float* sums, uint32_t first, uint32_t 
     const float v = *a;
     if (v != 0.0f) {
       *a = 0.0f;
-      atomic_add(dst + (size_t)sid[j] * stride + r, v);
+      atomic_add(dst + (size_t)id(j) * stride + r, v);
     }
   }
 }
 
-template <uint32_t kRow>
+template <uint32_t kRow, typename Id>
 __device__ __forceinline__ void bwd_flush_geometry(const RenderBwdParams& p, float* sums, uint32_t splats,
-                                                   const uint32_t* sid) {
-  bwd_flush<kRow, 9>(sums, kSumT, splats, sid, p.dtransmat, 9);
-  bwd_flush<kRow, 2>(sums, kSumM, splats, sid, p.dmean2D, 3);
-  bwd_flush<kRow, 3>(sums, kSumN, splats, sid, p.dnormal, 3);
-  bwd_flush<kRow, 1>(sums, kSumO, splats, sid, p.dopacity, 1);
-  if (p.dshapes != nullptr) bwd_flush<kRow, 1>(sums, kSumK, splats, sid, p.dshapes, 1);
+                                                   const Id& id) {
+  bwd_flush<kRow, 9>(sums, kSumT, splats, id, p.dtransmat, 9);
+  bwd_flush<kRow, 2>(sums, kSumM, splats, id, p.dmean2D, 3);
+  bwd_flush<kRow, 3>(sums, kSumN, splats, id, p.dnormal, 3);
+  bwd_flush<kRow, 1>(sums, kSumO, splats, id, p.dopacity, 1);
+  if (p.dshapes != nullptr) bwd_flush<kRow, 1>(sums, kSumK, splats, id, p.dshapes, 1);
 }
 
 constexpr int kBwdCand = 8;  // candidate splats a pixel holds between the test and the hit pass
@@ -919,8 +920,9 @@ __global__ void __launch_bounds__(kBwdThreads) render_backward_rgb_kernel(const 
       bwd_add_row<kSumColour>(hit, j, v, sums);
     }
     __syncthreads();
-    bwd_flush_geometry<kSumColour>(p, sums, n, sid);
-    bwd_flush<kSumColour, 3>(sums, kSumCol, n, sid, p.dcolors, 3);
+    const auto id_at = [&](uint32_t j) { return sid[j]; };
+    bwd_flush_geometry<kSumColour>(p, sums, n, id_at);
+    bwd_flush<kSumColour, 3>(sums, kSumCol, n, id_at, p.dcolors, 3);
     __syncthreads();
   }
 }
@@ -1118,14 +1120,18 @@ __device__ __forceinline__ void bwd_row_grads(const RenderBwdParams& p, bool on,
   }
 }
 
-// Three workgroups per CU (52.6 KB of LDS each) where the registers allow:
-// F <= 4 fits 168 VGPRs, F = 8 keeps two.
+// LDS of a CU, and the granules it is given out in.
+constexpr size_t kLdsPerCU = 160 * 1024, kLdsGranule = 1280;
+
+// Three workgroups per CU where the registers allow: F <= 4 fits 168 VGPRs,
+// F = 8 keeps two.  52.1 KB of LDS each, 42 granules of the 128: with the
+// splats' ids in an array of their own it was 43, two workgroups per CU, and
+// the 1M-splat step (1600x1064, F = 4) took 81.5 ms instead of 70.9.
 template <int F, int kRows>
 __global__ void __launch_bounds__(kBwdThreads) __attribute__((amdgpu_waves_per_eu(F <= 4 ? 3 : 2)))
 render_backward_kernel(const RenderBwdParams p) {
   constexpr int kMasks = kBwdBatch / 64;
   __shared__ float4 srec[kBwdChunks][kBwdBatch];
-  __shared__ uint32_t sid[kBwdBatch];
   __shared__ float sums[kBwdBatch * kSumHash];
   __shared__ float4 hq[kBwdWaves][kBwdQueue];       // (xyz, w), then (dot, dxyz)
   __shared__ uint16_t hmeta[kBwdWaves][kBwdQueue];  // owner lane | level count << 6
@@ -1134,6 +1140,9 @@ render_backward_kernel(const RenderBwdParams p) {
   __shared__ uint8_t lj[kBwdWaves][kBwdWide];
   __shared__ uint64_t smask[kBwdWaves][kMasks];
   __shared__ __attribute__((aligned(8))) uint32_t saux[kBwdWaves][kScatterAux];
+  constexpr size_t kLds = sizeof(srec) + sizeof(sums) + sizeof(hq) + sizeof(hmeta) + sizeof(noted) + sizeof(lact) +
+                          sizeof(lj) + sizeof(smask) + sizeof(saux);
+  static_assert(3 * ((kLds + kLdsGranule - 1) / kLdsGranule) * kLdsGranule <= kLdsPerCU, "three workgroups per CU");
 
   // level parts: workgroup b runs on XCD b % 8, dealt as in the forward
   uint32_t pos = blockIdx.x, part = 0u;
@@ -1168,6 +1177,7 @@ render_backward_kernel(const RenderBwdParams p) {
   __syncthreads();
   const uint32_t total = range.y - range.x;
   const uint32_t tlast = min(total, max(max(slast[0], slast[1]), max(slast[2], slast[3])));
+  const auto id_at = [&](uint32_t j) { return __float_as_uint(srec[6][j].w); };
 
   for (uint32_t below = tlast; below > 0u; below -= min(below, (uint32_t)kBwdBatch)) {
     const uint32_t n = min((uint32_t)kBwdBatch, below);
@@ -1179,7 +1189,7 @@ render_backward_kernel(const RenderBwdParams p) {
         const float4* rec = reinterpret_cast<const float4*>(p.records) + 8 * (size_t)id;
 #pragma unroll
         for (int c = 0; c < kBwdChunks; c++) srec[c][threadIdx.x] = rec[c];
-        sid[threadIdx.x] = id;
+        srec[6][threadIdx.x].w = __uint_as_float(id);  // the depth's slot: the backward recomputes depth per hit
         bb = rec[7];
       }
       bwd_block_masks<kMasks>(in, bb, tx, ty, wid, smask);
@@ -1213,7 +1223,7 @@ render_backward_kernel(const RenderBwdParams p) {
           T1 = T1 / (1.f - h.alpha);
           const float wgt = h.alpha * T1;
           float wt, xyz[3];
-          const uint32_t lane_levels = bwd_hit_levels<kRows>(p, h, srec[3][j], srec[4][j], srec[5][j], q6, sid[j], xyz, wt);
+          const uint32_t lane_levels = bwd_hit_levels<kRows>(p, h, srec[3][j], srec[4][j], srec[5][j], q6, id_at(j), xyz, wt);
           // the grid's share of the gradient: (1 - weight) of it in mode 12,
           // weight times it in mode 14
           const float hw = kRows == 2 ? wgt * (p.azero ? wt : 1.0f - wt) : wgt;
@@ -1280,7 +1290,7 @@ render_backward_kernel(const RenderBwdParams p) {
         if (on) {
           j = e & 255u;
           const float4 q1 = srec[1][j], q2 = srec[2][j], q3 = srec[3][j];
-          id = sid[j];
+          id = id_at(j);
           BwdHit h;
           bwd_hit(srec[0][j], q1, q2, px.pxf, px.pyf, p.beta, true, h, p.kernel_type, srec[6][j].z);
           px.T = px.T / (1.f - h.alpha);
@@ -1342,10 +1352,10 @@ render_backward_kernel(const RenderBwdParams p) {
       T1 = px.T;
     }
     __syncthreads();
-    bwd_flush_geometry<kSumHash>(p, sums, n, sid);
-    bwd_flush<kSumHash, 9>(sums, kSumH, n, sid, p.dhomo, 9);
-    bwd_flush<kSumHash, 1>(sums, kSumS, n, sid, p.gradsum, 1);
-    if constexpr (kRows == 2) bwd_flush<kSumHash, 1>(sums, kSumW, n, sid, p.dcolors + p.wslot, (uint32_t)p.cstride);
+    bwd_flush_geometry<kSumHash>(p, sums, n, id_at);
+    bwd_flush<kSumHash, 9>(sums, kSumH, n, id_at, p.dhomo, 9);
+    bwd_flush<kSumHash, 1>(sums, kSumS, n, id_at, p.gradsum, 1);
+    if constexpr (kRows == 2) bwd_flush<kSumHash, 1>(sums, kSumW, n, id_at, p.dcolors + p.wslot, (uint32_t)p.cstride);
     __syncthreads();
   }
 }
