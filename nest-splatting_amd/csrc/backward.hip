@@ -147,8 +147,8 @@ __device__ __forceinline__ void stage_flush(const uint32_t* st, uint32_t nb, flo
   wave_lds_order();
 }
 
-constexpr int kScatterAux = 128;   // dwords of LDS per wave beside the staging area
-constexpr uint32_t kFewCells = 8;  // mean lanes per cell above which cells are summed in registers
+constexpr int kScatterAux = 128;  // dwords of LDS per wave beside the staging area
+constexpr uint32_t kBigCell = 5;  // lanes of a cell from which they are summed in registers
 
 // Table gradient of one level for the wave (uniform control flow): lanes
 // whose hits fall in the same cell (same g) share all eight corner entries.
@@ -156,20 +156,30 @@ constexpr uint32_t kFewCells = 8;  // mean lanes per cell above which cells are 
 // cell; the lane that is left there, if its cell is the same, leads the lane's
 // cell (a lane that finds another cell there goes alone, which costs its
 // merging and nothing else).
-//  - Few cells (coarse levels: neighbouring pixels and splats adjacent in
-//    depth): a cell's 8F values are summed over its lanes with
-//    recursive-halving reduce-scatters, 16 values at a time (after one, lane l
-//    holds the sum of value l / 4 of the chunk), written straight to a staging
-//    slot; full sets of slots are added with packed atomics.
-//  - Otherwise the cells are numbered, and one x-pair of corners at a time the
-//    leaders write their 2F values to their cell's slot, the other lanes add
-//    theirs there (LDS atomics) and the slots are added to memory, consecutive
-//    values by consecutive lanes, so that an x-pair of entries is one request
-//    where it lies in one 64-byte segment.
-// Finding the cells one at a time by ballots and summing the small ones by
-// pointer jumping took 8.6 ms a step with feature rows (401x399, 3 levels),
-// where this takes 7.5; at 16 levels (801x517) both wait for the atomics.
-template <int F>
+//  - Cells of kBigCell lanes or more (neighbouring pixels and splats adjacent
+//    in depth) one after the other: the 8F values are summed over the cell's
+//    lanes with recursive-halving reduce-scatters, 16 values at a time (after
+//    one, lane l holds the sum of value l / 4 of the chunk), and written
+//    straight to a staging slot; full sets of slots are added with packed
+//    atomics.
+//  - The others are numbered, and one x-pair of corners at a time the leaders
+//    write their 2F values to their cell's slot, the other lanes add theirs
+//    there (LDS atomics) and the slots are added to memory, consecutive values
+//    by consecutive lanes, so that an x-pair of entries is one request where it
+//    lies in one 64-byte segment.
+// LDS adds to one address run one after the other, so the line between the two
+// is a cell's own size.  Training steps, ms, summed in registers from 5 / 9 / 13
+// / 21 lanes: 1M splats in contracted space, 16 levels of 4 (6 lanes a cell)
+// 57.8 / 61.6 / 73.8 / 94.1; 1M on a shell, 16 of 2, 60.7 / 61.0 / 61.0 / 61.4;
+// feature rows at 401x399, 3 of 4, 7.32 / 7.32 / 7.42 / 7.50; from 4 lanes
+// within 1% of 5.  By the wave's mean (more than 8 lanes a cell) the first was
+// 70.9.  Finding the cells one at a time by ballots and summing the
+// small ones by pointer jumping: 58.5, 62.1 and 8.5.
+// kTight: the caller's registers are short, so one read ahead of its add and
+// smaller chunks (feature rows with F = 4: mode 4, 142,648 splats at 800x800, 3
+// levels, 9.7 ms against 10.4; mode 12, 1M splats, 30.0 against 33.2).  Elsewhere
+// it is the slower: 8 levels of 8, 33.7 ms against 33.1.
+template <int F, bool kTight>
 __device__ __forceinline__ void scatter_level(bool on, const uint32_t gc[3], const uint32_t idx[8], const float* cv,
                                               float* dl, uint32_t* st, uint32_t* aux) {
   constexpr int NV = 8 * F;
@@ -193,20 +203,35 @@ __device__ __forceinline__ void scatter_level(bool on, const uint32_t gc[3], con
   }
   const bool lead = on && ld == lane;
   uint64_t leaders = __ballot(lead);
-  const uint32_t cells = (uint32_t)__popcll(leaders);
   wave_lds_order();
-  if ((uint32_t)__popcll(onm) > cells * kFewCells) {
+  const bool shared = leaders != onm;  // some cell has more than one lane
+  if (shared) {
+    // lanes of each cell, counted at its leader's place (not worth its two
+    // round trips where cells have fewer than 2 lanes on average)
+    uint64_t big = 0ull;
+    if ((uint32_t)__popcll(onm) >= 2u * (uint32_t)__popcll(leaders)) {
+      aux[lane] = 0u;
+      wave_lds_order();
+      if (on) __hip_atomic_fetch_add(aux + ld, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      wave_lds_order();
+      big = __ballot(lead && aux[lane] >= kBigCell);
+      wave_lds_order();
+    }
+    leaders &= ~big;
+    const bool in_big = on && ((big >> ld) & 1ull) != 0ull;
+    on = on && !in_big;
     uint32_t nb = 0u;  // staging slots in use
-    while (leaders != 0ull) {
-      const int l0 = __ffsll((long long)leaders) - 1;
-      leaders &= leaders - 1ull;
-      const bool mem = on && ld == (uint32_t)l0;
+    while (big != 0ull) {
+      const int l0 = __ffsll((long long)big) - 1;
+      big &= big - 1ull;
+      const bool mem = in_big && ld == (uint32_t)l0;
       if (nb == kSlots) {
         stage_flush<F>(st, nb, dl);
         nb = 0u;
       }
       // reduce-scatter in chunks of kCh values (fewer live registers)
-      constexpr int kCh = NV < 16 ? NV : 16;
+      constexpr int kMost = kTight ? 8 : 16;
+      constexpr int kCh = NV < kMost ? NV : kMost;
       constexpr int kRepC = 64 / kCh;
 #pragma unroll
       for (int c = 0; c < NV / kCh; c++) {
@@ -237,15 +262,15 @@ __device__ __forceinline__ void scatter_level(bool on, const uint32_t gc[3], con
       if (lane < 8u) st[kIdx + nb * 8u + lane] = e;
       nb++;
     }
-    stage_flush<F>(st, nb, dl);
-    wave_lds_order();
-    return;
+    if (nb > 0u) stage_flush<F>(st, nb, dl);
   }
+  const uint32_t cells = (uint32_t)__popcll(leaders);
   constexpr uint32_t kPair = 2 * F;                                   // values of an x-pair of corners
   constexpr uint32_t kCells = 256u / kPair < 64u ? 256u / kPair : 64u;  // cells whose pairs fit the staging area
   const uint32_t rank = (uint32_t)__popcll(leaders & ((1ull << lane) - 1ull));
   const uint32_t cell = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(ld << 2), (int)rank);
   float* sums = reinterpret_cast<float*>(st);
+  constexpr uint32_t kRounds = kCells * kPair / 64u;
   for (uint32_t c0 = 0; c0 < cells; c0 += kCells) {
     const uint32_t slot = cell - c0;  // past kCells for the cells before c0
     const bool in = on && slot < kCells;
@@ -259,15 +284,34 @@ __device__ __forceinline__ void scatter_level(bool on, const uint32_t gc[3], con
         *reinterpret_cast<uint2*>(aux + 2u * slot) = make_uint2(idx[2 * c], idx[2 * c + 1]);
       }
       wave_lds_order();
-      if (in && !lead) {
+      if (shared) {
+        if (in && !lead) {
 #pragma unroll
-        for (uint32_t i = 0; i < kPair; i++) lds_add(sums + slot * kPair + i, cv[c * kPair + i]);
+          for (uint32_t i = 0; i < kPair; i++) lds_add(sums + slot * kPair + i, cv[c * kPair + i]);
+        }
+        wave_lds_order();
       }
-      wave_lds_order();
-      for (uint32_t f = lane; f < nval; f += 64u) {
-        const float val = sums[f];
-        const uint32_t e = aux[f / F];
-        if (val != 0.0f) atomic_add(dl + (size_t)e * F + (f % F), val);
+      if constexpr (kTight) {
+        for (uint32_t f = lane; f < nval; f += 64u) {
+          const float val = sums[f];
+          const uint32_t e = aux[f / F];
+          if (val != 0.0f) atomic_add(dl + (size_t)e * F + (f % F), val);
+        }
+      } else {
+        // all reads in flight together; what lies past nval is left of other cells
+        float val[kRounds];
+        uint32_t e[kRounds];
+#pragma unroll
+        for (uint32_t r = 0; r < kRounds; r++) {
+          const uint32_t f = 64u * r + lane;
+          val[r] = sums[f];
+          e[r] = aux[f / F];
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < kRounds; r++) {
+          const uint32_t f = 64u * r + lane;
+          if (f < nval && val[r] != 0.0f) atomic_add(dl + (size_t)e[r] * F + (f % F), val[r]);
+        }
       }
       wave_lds_order();
     }
@@ -279,7 +323,7 @@ __device__ __forceinline__ void scatter_level(bool on, const uint32_t gc[3], con
 // dot = sum_ch feat[ch] * dpix[ch], adds w_corner * w * dpix to the table at
 // every corner of every level below lane_levels, and returns dL/dxyz
 // (hashgrid.h:213-299; grad_scale of :66-97).
-template <int F>
+template <int F, bool kTight>
 __device__ __forceinline__ void hash_backward_wave(const GridParams& g, nest_i32x4 rsrc, const float u[3],
                                                    float grad_scale, uint32_t lane_levels, float w,
                                                    const float* dpix, size_t HW, float* dtable, uint32_t* st, uint32_t* aux,
@@ -361,7 +405,7 @@ __device__ __forceinline__ void hash_backward_wave(const GridParams& g, nest_i32
         for (int f = 0; f < F; f++) dxyz[gd] += gf[f] * rg[f];
       }
     }
-    scatter_level<F>(on, gc, cn.idx, cv, dtable + (size_t)lv.base[l] * F, st, aux);
+    scatter_level<F, kTight>(on, gc, cn.idx, cv, dtable + (size_t)lv.base[l] * F, st, aux);
   }
 }
 
@@ -1262,8 +1306,9 @@ render_backward_kernel(const RenderBwdParams p) {
         float dot, dxyz[3];
         // the chunk's queue entries (read above, rewritten below) stage the
         // table-gradient atomics meanwhile
-        hash_backward_wave<F>(g, rsrc, u, gsc, lev, w, dp, HW, p.dtable, reinterpret_cast<uint32_t*>(&hq[wid][r0]),
-                              saux[wid], part, p.parts, dot, dxyz);
+        hash_backward_wave<F, kRows != 0 && F == 4>(g, rsrc, u, gsc, lev, w, dp, HW, p.dtable,
+                                                    reinterpret_cast<uint32_t*>(&hq[wid][r0]), saux[wid], part,
+                                                    p.parts, dot, dxyz);
         if (on) hq[wid][e] = make_float4(dot, dxyz[0], dxyz[1], dxyz[2]);
       }
       __builtin_amdgcn_wave_barrier();
@@ -1648,7 +1693,7 @@ __global__ void __launch_bounds__(256) grid_encode_backward_kernel(const GridEnc
       }
     }
   }
-  scatter_level<F>(on, gc, cn.idx, cv, p.grad_table + (size_t)p.lv.base[l] * F, stage[wid], saux[wid]);
+  scatter_level<F, false>(on, gc, cn.idx, cv, p.grad_table + (size_t)p.lv.base[l] * F, stage[wid], saux[wid]);
 }
 
 // kernel_input_backward (gridencoder.cu:316-366) with the dy_dx of kernel_grid

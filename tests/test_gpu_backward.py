@@ -250,6 +250,32 @@ def test_grid_encode_backward_cells(oracle, F, B, spread):
     assert _rel(xt.grad.cpu().numpy(), gi) < TOL
 
 
+@pytest.mark.parametrize("F", [1, 2, 4, 8])
+@pytest.mark.parametrize("sizes", [[4] * 16, [5] * 12 + [4], [1] * 60 + [4], [3] * 21 + [1], [6] * 10 + [2] * 2, [59, 5],
+                                   [60, 4], [30, 9, 6, 5, 4, 4, 3, 2, 1], [1] * 59 + [5]])
+def test_grid_encode_backward_cell_sizes(oracle, F, sizes):
+    """Waves of 64 points whose cells at the finest level hold the listed
+    numbers of points: on both sides of the size from which a cell is summed in
+    registers, alone and mixed.  As above: each entry is a short sum."""
+    from gridencoder import GridEncoder
+    assert sum(sizes) == 64
+    rng = np.random.default_rng(F)
+    enc = GridEncoder(3, 4, F, 2.0, 16, 13).to(DEV)
+    res = 16 * 2 ** 3
+    waves = []
+    for _ in range(9):
+        cell = np.repeat(rng.integers(8, res - 8, (len(sizes), 3)), sizes, axis=0)
+        waves.append(rng.permutation((cell + rng.uniform(0.2, 0.8, (64, 3))) / res))
+    x = np.concatenate(waves).astype(np.float32)
+    y = enc(_t(x))
+    g = rng.standard_normal(tuple(y.shape)).astype(np.float32)
+    y.backward(_t(g))
+    tab = enc.embeddings.detach().cpu().numpy()
+    grid = oracle.make_grid(4, F, 1.0, 16, enc._offsets_host, tab, (0.0, 1.0), False)
+    gt, _ = oracle.grid_encode_backward(grid, x, g)
+    assert _rel(enc.embeddings.grad.cpu().numpy(), gt) < TOL
+
+
 @pytest.mark.parametrize("rows", [4920, 4921, 8193, 40003])
 @pytest.mark.parametrize("shift", [0, 1, 2, 3])
 def test_gradient_zeroed_at_any_alignment(rows, shift):
