@@ -34,6 +34,7 @@ NotImplementedError instead of returning zeros.
 """
 from __future__ import annotations
 
+from dataclasses import replace
 from typing import NamedTuple
 
 import numpy as np
@@ -224,7 +225,10 @@ class _RasterizeGaussians(torch.autograd.Function):
         ctx.num_rendered = res.num_rendered
         ctx.render_mode = render_mode
         ctx.kernel_type = int(kernel_type)
-        ctx.fw = dict(res=res, settings=settings, grid=grid, C=C, colors=colors,
+        # without the tensors returned below: an output kept here would hold its own
+        # graph, and nothing would free the step's memory
+        kept = replace(res, color=None, others=None, radii=None, trans_avg=None, cover_pixels=None)
+        ctx.fw = dict(res=kept, settings=settings, grid=grid, C=C, colors=colors,
                       shapes=None if kernel_type == 0 else shapes.detach().reshape(-1),
                       shs=None if (level > 0 or colors is not None or _empty(sh)) else sh.detach(),
                       sh_degree=int(raster_settings.sh_degree),

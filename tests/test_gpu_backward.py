@@ -385,3 +385,37 @@ def test_autograd_kernel_type_through_drop_in_rasterizer():
                      (scales.grad, gb.dscales), (rots.grad, gb.drotations)]:
         err = _rel(got.cpu().numpy(), ref.cpu().numpy())
         assert err < 1e-5, err
+
+
+def test_training_step_gives_its_memory_back(oracle):
+    """What a step allocates is free once its outputs and gradients are, without
+    a run of the cycle collector."""
+    import gc
+
+    from diff_surfel_rasterization import GaussianRasterizer, GaussianRasterizationSettings, HashGridSettings
+    sc = scene("cfg1")
+    cam = sc.cameras[0]
+    rs = GaussianRasterizationSettings(
+        image_height=cam.image_height, image_width=cam.image_width, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy,
+        bg=torch.zeros(3, device=DEV), scale_modifier=1.0, viewmatrix=cam.world_view_transform,
+        projmatrix=cam.full_proj_transform, sh_degree=0, campos=cam.camera_center, prefiltered=False, debug=False,
+        beta=0.0, if_contract=False, record_transmittance=False)
+    hs = HashGridSettings(L=0, S=0.0, H=0, align_corners=False, interpolation=0, shape_dims=torch.tensor([0, 3, 3]))
+    ras = GaussianRasterizer(rs, hs)
+    means, colors = _t(sc.means).requires_grad_(True), torch.rand((sc.means.shape[0], 3), device=DEV)
+
+    def step():
+        color, _, allmap, _, _ = ras(means, torch.zeros_like(means), _t(sc.opacity), colors_precomp=colors,
+                                     scales=_t(sc.scales), rotations=_t(sc.rotations))
+        return torch.autograd.grad(color.sum() + allmap[1].sum(), means)[0].abs().sum().item()
+
+    assert step() > 0
+    gc.collect()
+    gc.disable()
+    try:
+        held = torch.cuda.memory_allocated()
+        for _ in range(3):
+            step()
+        assert torch.cuda.memory_allocated() <= held
+    finally:
+        gc.enable()
