@@ -1464,17 +1464,24 @@ hipError_t launch_render(const RenderParams& p, hipStream_t s) {
 // parts repeat the compositing (0.4 of the 2.8 ms of the 100k-splat 800 x 800
 // frame) and split the lookups, each XCD keeping to one part's tables.  The
 // levels are dealt round-robin because the fine ones cost most (contiguous
-// halves: 3.70 ms where the dealt ones take 2.33).  Measured, render ms with
-// 1 / 2 / 4 / 8 parts, 16 levels: 64 tiles 0.94 / 0.69 / 0.57 / 0.49; 256
-// tiles 1.11 / 0.79 / 0.70 / 0.95; 625 tiles 1.32 / 1.02 / 1.25 / 1.91 and 1.66
-// / 1.48 / 1.55 / 2.17; 1200 tiles 2.03 / 1.80 / 2.19; 2500 tiles 2.91 / 2.33 /
-// 2.71 (object), 2.28 / 2.35 / 3.06 and 2.99 / 2.72 / 3.42 (unbounded); 4056
-// tiles 3.60 / 3.90 / 5.34.  8 levels: 64 tiles 0.68 / 0.55 / 0.48 / 0.47; 256
-// tiles 0.70 / 0.58 / 0.55 / 0.88; 625 tiles 0.71 / 0.63 / 0.99; 1200 tiles
-// 0.94 / 1.08 / 1.61.
+// halves: 3.70 ms where the dealt ones take 2.33).  Whole frames over one part,
+// geometric mean and worst of six scenes (300 and 3,000 wide faint splats, the
+// same opaque, 30k, 200k in contracted space), F = 2 and 4, with 2 / 4 / 8 parts:
+//   16 levels: 100 tiles 0.68 / 0.55 / 0.49 (0.78 / 0.68 / 0.63); 320 0.81 / 0.81 /
+//   0.78 (0.85 / 1.03 / 1.21); 414 0.80 / 0.76 / 0.79; 600 0.85 / 0.78 (0.96 /
+//   1.04); 1200 0.84 / 0.81 (0.89 / 1.02); 2500 0.85 / 0.86 (0.95 / 1.20); 3072
+//   0.88 / 0.94 (1.04 / 1.34); 4056 (1M splats) 1.08 / 1.48.  12 levels: 2500 0.85
+//   (1.03); 3072 0.91 (1.10).
+//   8 levels: 256 tiles 0.80 / 0.76 (0.91 / 0.93); 320 0.83 / 0.91 (0.87 / 1.19); 600
+//   0.89 / 0.94 (1.08 / 1.33); 1200 0.90 (1.07); 2500 0.92 (1.15).
+//   5 levels: 100 tiles 0.85 / 0.75; 256 0.85 / 0.84 (0.90 / 1.02); 320 0.88 / 1.06;
+//   414 0.89 (0.92); 600 1.00 (1.15 in contracted space; 200k on a shell 0.91).  4
+//   levels: 100 tiles 0.80 / 0.77; 256 0.81 / 0.87 (0.86 / 1.10); 320 0.84 / 1.11;
+//   600 0.95 (1.07; 200k on a shell 0.85); 770 1.00 (1.15).
 static uint32_t level_parts(uint32_t tiles, uint32_t L) {
   if (L > 8u) return tiles <= 96u ? 8u : tiles <= 400u ? 4u : tiles <= 2560u ? 2u : 1u;
-  if (L >= 4u) return tiles <= 320u ? 4u : tiles <= 768u ? 2u : 1u;
+  if (L > 4u) return tiles <= 256u ? 4u : tiles <= 768u ? 2u : 1u;
+  if (L == 4u) return tiles <= 128u ? 4u : tiles <= 768u ? 2u : 1u;
   return 1u;
 }
 

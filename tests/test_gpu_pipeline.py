@@ -324,12 +324,14 @@ def test_kernel_types_parity(oracle, name, kt):
 
 
 # (W, H, L, F, half table): tile counts on both sides of each line of the
-# level-parts rule (96, 400 and 2560 tiles over 8 levels, 320 and 768 up to
-# 8), level counts that the parts do not divide, and 2 levels (no parts)
+# level-parts rule (96, 400 and 2560 tiles over 8 levels, 256 and 768 from 5 to
+# 8, 128 and 768 at 4), level counts that the parts do not divide, and 2 levels
+# (no parts)
 PART_CASES = [(96 * 16, 16, 16, 2, False), (97 * 16 - 3, 13, 11, 4, False), (20 * 16, 20 * 16, 9, 4, True),
               (401 * 16 - 15, 9, 16, 2, False), (64 * 16, 40 * 16, 13, 1, False), (197 * 16, 13 * 16 - 7, 16, 2, False),
               (320 * 16, 16, 8, 2, False), (321 * 16, 15, 5, 4, False), (96 * 16, 8 * 16, 7, 2, True),
-              (769 * 16, 10, 8, 4, True), (40, 24, 4, 2, False), (40, 24, 2, 4, False), (1, 1, 16, 4, False)]
+              (769 * 16, 10, 8, 4, True), (128 * 16, 16, 4, 2, False), (129 * 16 - 3, 13, 4, 4, True),
+              (256 * 16, 11, 7, 4, False), (257 * 16 - 9, 9, 5, 2, False), (40, 24, 4, 2, False), (40, 24, 2, 4, False), (1, 1, 16, 4, False)]
 
 
 @pytest.mark.parametrize("W,H,L,F,half", PART_CASES)
