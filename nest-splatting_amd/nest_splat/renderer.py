@@ -444,9 +444,10 @@ def _render_hybrid(cam, pc, pipe, bg_color, scaling_modifier, ingp, beta, max_in
 
 
 def _ops_followed() -> bool:
-    """Whether a trace, transform or mode may follow tensor operations.  torch
-    has no public names for some of these; without them the answer is yes."""
-    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+    """Whether a trace, transform or mode may follow tensor operations, or
+    autocast round them.  torch has no public names for some of these; without
+    them the answer is yes."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_autocast_enabled():
         return True
     try:
         return (torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None or

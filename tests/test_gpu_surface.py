@@ -119,3 +119,20 @@ def test_surface_maps_of_another_device_keep_the_general_path(monkeypatch):
     out = renderer.surface_maps(cam, a)
     monkeypatch.undo()
     np.testing.assert_array_equal(out["surf_depth"].cpu().numpy(), renderer.surface_maps(cam, a)["surf_depth"].cpu().numpy())
+
+
+def test_surface_maps_under_autocast_keep_the_general_path():
+    """Autocast rounds the products of the tensor operations: types and values
+    are theirs."""
+    from nest_splat.camera import look_at
+    from nest_splat.renderer import surface_maps
+    W, H = 33, 20
+    cam = look_at((0.4, -3.0, 1.0), (0, 0, 0), 50.0, W, H)
+    a = _allmap(W, H, 8).to(DEV)
+    for dtype in (torch.float16, torch.bfloat16):
+        with torch.autocast("cuda", dtype=dtype), torch.no_grad():
+            out = surface_maps(cam, a)
+            general = surface_maps(cam, a.permute(0, 2, 1).contiguous().permute(0, 2, 1))
+        for k, v in general.items():
+            assert out[k].dtype == v.dtype, k
+        assert out["rend_normal"].dtype == dtype
