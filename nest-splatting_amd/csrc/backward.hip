@@ -1768,14 +1768,22 @@ hipError_t launch_grid_encode_backward(const GridEncodeBwdParams& p, hipStream_t
 // tiles leave the chip idle behind each wave's chain of hits, levels and
 // scatter steps.  Repeating the hit and recursion passes costs more than it
 // gives once the tiles fill the chip and the atomics bound the launch.  Whole
-// backward, ms with 1 / 2 / 4 / 8 parts, 16 levels: 64 tiles 8.3 / 4.6 / 2.7 /
-// 1.8; 256 tiles 4.21 / 2.48 / 1.68 / 1.92; 625 tiles 11.5 / 7.2 / 7.6 / 8.2;
-// 1683 tiles 21.9 / 20.5 / 20.9 / 22.9 and 26.7 / 23.9 / 24.1 / 28.0; 4056
-// tiles 39.8 / 38.9 / 44.3 and 41.9 / 43.3 / 56.3.  3 levels: 256 tiles 1.39 /
-// 1.07 / 1.04; 676 tiles with feature rows 6.8 / 6.9; 1683 tiles 6.9 / 9.4.
+// training steps over one part, geometric mean and worst of three scenes (3,000
+// wide faint splats, 2,000 in a cube, 200k in contracted space), F = 2 and 4, with
+// 2 / 4 / 8 parts:
+//   16 levels: 16 tiles 0.63 / 0.45 / 0.36; 100 0.62 / 0.45 / 0.40; 256 0.74 / 0.74 /
+//   0.75 (0.86 / 0.83 / 0.85); 414 0.94 / 0.95 / 0.96 (0.99 / 1.04 / 1.07); 600 1.00 /
+//   0.97 (1.08 / 1.07); 1683 0.99 / 1.01; 2500 0.99 / 1.01; 3600 1.00 / 1.03.
+//   8 levels: 100 tiles 0.68 / 0.53 / 0.46; 256 0.78 / 0.80 (0.86 / 0.87); 320 0.91 /
+//   1.02 (0.99 / 1.15); 600 1.01 / 1.03 (1.14 in contracted space, 0.93 in the cube);
+//   1200 0.99 / 1.01.
+//   4 levels: 100 tiles 0.75 / 0.63; 256 0.80 / 0.80 (0.83 / 0.93); 320 0.93 / 1.06
+//   (1.00 / 1.24); 600 1.00 / 1.08.
+//   Feature rows, 3 levels: 100 tiles 0.90; 256 0.92; 320 1.01 (1.06); 600 1.23 (1.42).
+//   2 levels: 256 0.85; 320 0.92 (1.01); 600 1.12.
 static uint32_t bwd_level_parts(uint32_t tiles, uint32_t L) {
   if (L > 8u) return tiles <= 96u ? 8u : tiles <= 400u ? 4u : tiles <= 2560u ? 2u : 1u;
-  if (L >= 4u) return tiles <= 320u ? 4u : tiles <= 768u ? 2u : 1u;
+  if (L >= 4u) return tiles <= 256u ? 4u : tiles <= 768u ? 2u : 1u;
   return L >= 2u && tiles <= 320u ? 2u : 1u;
 }
 

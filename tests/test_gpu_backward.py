@@ -147,8 +147,8 @@ def test_backward_hash_parity(oracle, name):
 
 
 # (path, W, H, L, F, log scale): tile counts on both sides of each line of the
-# backward's level-parts rule (96, 400 and 2560 tiles over 8 levels; 320 and
-# 768 below), level counts the parts do not divide, and on the 3-channel path
+# backward's level-parts rule (96, 400 and 2560 tiles over 8 levels; 256 and
+# 768 from 4 to 8; 320 below), level counts the parts do not divide, and on the 3-channel path
 # splats of a pixel and of many waves (few and many lanes at one splat), with
 # several batches per tile.  The wide frames' splats cover thousands of pixels
 # (a 50 degree view 6,401 pixels wide), so a coarse level's row or a splat's scale
@@ -159,6 +159,7 @@ def test_backward_hash_parity(oracle, name):
 EDGE_TOL = 1e-4
 EDGE_CASES = [("hash", 96 * 16, 16, 16, 2, -3.0), ("hash", 97 * 16 - 3, 13, 11, 4, -3.0),
               ("hash", 401 * 16 - 15, 9, 16, 2, -3.0), ("hash", 2561 * 16, 5, 9, 1, -3.0),
+              ("hash", 256 * 16, 9, 7, 2, -3.0), ("hash", 257 * 16, 9, 5, 4, -3.0),
               ("hash", 321 * 16, 9, 5, 2, -3.0), ("hash", 769 * 16, 7, 8, 4, -3.0), ("hash", 40, 24, 2, 4, -2.0),
               ("hash", 17, 33, 16, 2, -4.5), ("sh", 40, 24, 1, 2, -2.0), ("sh", 17, 33, 1, 2, -5.5),
               ("sh", 400, 16, 1, 2, -3.5)]

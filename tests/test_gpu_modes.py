@@ -665,7 +665,7 @@ def _adaptive_backward(oracle, mode, sc, total, hyb, gl, kt, tol):
 
 # (render mode, W, H, total levels, per-splat levels, grid levels, F): the
 # backward's level parts with feature rows, on both sides of the rule's lines
-# (320 tiles below 4 levels, 320 and 768 up to 8, 2560 beyond), so that the
+# (320 tiles below 4 levels, 256 and 768 up to 8, 2560 beyond), so that the
 # rows' gradients and products are sent by part 0 of several workgroups and by
 # a tile's only one; and an ordinary frame with one workgroup per tile.  The
 # wide frames' splats cover thousands of pixels (a 50 degree view up to 40,976
@@ -674,7 +674,7 @@ def _adaptive_backward(oracle, mode, sc, total, hyb, gl, kt, tol):
 # float32 sum errs by about u sqrt(n) = 6e-5 of its largest partial sum, on
 # both sides: 1e-4.
 ROW_EDGE_TOL = 1e-4
-ROW_EDGE_CASES = [(4, 320 * 16, 9, 5, 2, 3, 8), (4, 321 * 16, 9, 8, 5, 3, 4), (4, 768 * 16 - 5, 7, 8, 3, 5, 2),
+ROW_EDGE_CASES = [(4, 256 * 16, 9, 7, 2, 5, 4), (12, 257 * 16, 9, 8, 2, 6, 2), (4, 320 * 16, 9, 5, 2, 3, 8), (4, 321 * 16, 9, 8, 5, 3, 4), (4, 768 * 16 - 5, 7, 8, 3, 5, 2),
                   (4, 769 * 16, 7, 13, 5, 8, 4), (4, 2560 * 16, 5, 12, 2, 10, 2), (4, 2561 * 16, 5, 12, 3, 9, 4),
                   (4, 401, 399, 6, 3, 3, 4), (12, 320 * 16, 9, 6, 3, 3, 8), (12, 321 * 16, 9, 6, 3, 3, 4),
                   (12, 768 * 16, 7, 8, 2, 6, 4), (12, 769 * 16 - 3, 7, 7, 3, 4, 8), (12, 2561 * 16, 5, 12, 3, 9, 2),
