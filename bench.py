@@ -54,10 +54,9 @@ def render_compulsory_bound(P: int, NR: int, HW: int, table_bytes: int, C: int) 
 # What bounds the render kernel, from its counters (TA busy, L1 accesses per
 # clock, VALU share): the 16-byte table gathers' vector-L1 address and tag
 # rate and the latency of the gathers that miss L2.
-RENDER_LIMITER = ("the lookup drains' instruction stream: VALU issue ~0.63 and the texture addresser ~0.75 busy on "
-                  "the 1M-splat frame (one L1 tag access per CU clock); with every gather L1-resident the render "
-                  "takes 0.90x its time, without the drains 0.24x; HBM traffic is the counter-measured fetch + "
-                  "write")
+RENDER_LIMITER = ("the lookup drains' instruction stream: VALU issue 0.62 and the texture addresser 0.78 busy on "
+                  "the 1M-splat frame (one L1 tag access per CU clock, 2.7 waves a SIMD); without the drains the "
+                  "render takes 0.18x its time; HBM traffic is the counter-measured fetch + write")
 
 
 def load_counters(path: str) -> dict:

@@ -810,7 +810,10 @@ __device__ __forceinline__ void bwd_flush_geometry(const RenderBwdParams& p, flo
   if (p.dshapes != nullptr) bwd_flush<kRow, 1>(sums, kSumK, splats, id, p.dshapes, 1);
 }
 
-constexpr int kBwdCand = 8;  // candidate splats a pixel holds between the test and the hit pass
+// Candidate splats a pixel holds between the test and the hit pass (whole SH
+// training steps with 4 / 16 over 8: 200k small splats at 400x400 1.07 / 0.99, at
+// 800x800 1.00 / 1.02, others within 1%).
+constexpr int kBwdCand = 8;
 constexpr int kBwdWaves = kBwdThreads / 64;
 
 // Masks of the staged splats whose acceptance bbox meets each wave's 16 x 4
@@ -839,7 +842,11 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
 
-constexpr uint32_t kWideSplat = 24;  // candidate lanes from which a splat is taken by the whole wave
+// Candidate lanes from which a splat is taken by the whole wave.  Whole SH
+// training steps with 12 / 40 / never over 24: 200k splats at 800x800 0.99 / 1.03 /
+// 0.97, 3,000 wide faint ones at 400x400 0.97 / 1.03 / 1.05, 200k small ones at
+// 400x400 1.06 / 1.00 / 0.86.
+constexpr uint32_t kWideSplat = 24;
 
 // Colour path with 3 channels (SH colours, RGB).  A wave lists each pixel's
 // candidates (splats whose bbox meets its block, in front of the pixel's last
@@ -1072,9 +1079,10 @@ __global__ void __launch_bounds__(kBwdThreads) render_backward_colour_kernel(con
 //     wide splats make up the segment, the wave goes splat by splat), with the
 //     blending recursion and the gradients into the batch's LDS sums.
 // Whole kernel, ms, lockstep walk / this: 150k splats, 801x517, 16 levels F=2
-// 22.3 / 20.3 (3.4e8 atomic requests, ~17 of the ~20 G/s random adds reach);
-// 1M splats, 1600x1064, F=4 54.6 / 50.8 (8.7e8 requests); 60k splats with
-// 24-float rows blended with 3 levels, 401x399, 10.1 / 7.1.
+// 22.3 / 19.3 (3.3e8 atomic requests, 17.4 of the 20.9 G/s that random adds reach);
+// 1M splats, 1600x1064, F=4 54.6 / 51.1 (8.7e8 requests, 17.1 G/s); 60k splats with
+// 24-float rows blended with 3 levels, 401x399, 10.1 / 6.1 (0.7 waves a SIMD: 650
+// tiles are one round).
 // Frames of few tiles deal the levels round-robin over several workgroups per
 // tile (bwd_level_parts): everything the recursion sends out is linear in
 // (dot, dxyz) and the other loss terms, so each part sends its own levels'
@@ -1114,9 +1122,14 @@ __device__ __forceinline__ uint32_t bwd_hit_levels(const RenderBwdParams& p, con
 
 constexpr int kBwdQueue = 256;  // queued grid hits per wave
 constexpr int kBwdBatch = 128;  // splats staged per batch
-constexpr int kBwdNoted = 8;    // hits a lane notes per segment
-constexpr uint32_t kBwdWideLanes = 16;  // lanes per splat from which they are
+// Hits a lane notes per segment: with 4, feature rows at 401x399 take 1.05 and 200k
+// small splats at 400x400 1.08 times as long; 16 leave no LDS for three workgroups.
+constexpr int kBwdNoted = 8;
 constexpr int kBwdWide = 16;    // splats of a segment whose hits may be taken splat by splat
+// Lanes per splat from which they are.  Whole steps with 8 / 32 / never over 16:
+// feature rows at 401x399 1.03 / 1.02 / 1.01, 30k splats with rows at 400x400 1.00 /
+// 1.05 / 1.09, without rows within 1.5%.
+constexpr uint32_t kBwdWideLanes = 16;
 
 // A splat row's gradient on the leading n channels for the lanes with a hit,
 // coef * dL/dpixel_c (coefficient a below channel split, b from it on).  Lanes
@@ -1659,8 +1672,8 @@ __device__ __forceinline__ bool encode_outside(const float u[3]) {
 // feature was 8F requests per point and level; the scatter's instructions
 // carry whole x-pairs of entries, ~4.5 requests per cell, and points of one
 // cell are summed first.  142,648 random points on 16 levels of 2^19 entries,
-// F = 2: 2218 -> 660 us (490 at that rate); a step of 2,000,000 points in image
-// order: 82 -> 2.1 ms.  Levels over the grid's y: a wave's scatter is a serial
+// F = 2: 2218 -> 643 us (490 at that rate); a step of 2,000,000 points in image
+// order: 82 -> 2.0 ms.  Levels over the grid's y: a wave's scatter is a serial
 // chain, and 142,648 points alone are two waves per SIMD.
 template <int F>
 __global__ void __launch_bounds__(256) grid_encode_backward_kernel(const GridEncodeBwdParams p) {

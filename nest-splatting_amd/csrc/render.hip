@@ -58,7 +58,11 @@ constexpr int kRenderThreads = 256;
 constexpr int kBatch = 256;    // splats staged in LDS per batch
 constexpr int kRecChunks = 7;  // float4 chunks of the record staged per splat (the bbox, chunk 7, stays in registers)
 constexpr int kQueue = 4;      // pending hash lookups per pixel
-constexpr int kList = 8;       // candidate splats a pixel holds between the test and the hit pass
+// Candidate splats a pixel holds between the test and the hit pass.  Whole
+// frames with 4 / 16 entries over 8: 2,000 splats at 128x128 1.05 / 1.00, feature
+// rows at 800x800 1.04 / 1.22, 400k SH-coloured splats at 1237x822 1.03 / 1.04,
+// 1M and 4M splats 1.00-1.01 both; 200k small splats at 400x400 1.08 / 0.97.
+constexpr int kList = 8;
 constexpr int kWaveLanes = 64;
 constexpr int kWaves = kRenderThreads / kWaveLanes;
 
@@ -729,14 +733,14 @@ __device__ __forceinline__ void surface_accumulate(const RenderParams& p, const 
   }
 }
 
-// LDS (32 KB of staged records + 17 KB of queue) allows three workgroups per
-// CU; amdgpu_waves_per_eu(3) gives the matching 168-VGPR budget, which holds
-// 64 accumulators and eight in-flight 16-byte corner loads.
+// LDS (28 KB of staged records, 17 KB of queue, 2 KB of lists: 47.4 KB) allows
+// three workgroups per CU; amdgpu_waves_per_eu(3) gives the matching 168-VGPR
+// budget, which holds 64 accumulators and eight in-flight 16-byte corner loads.
 //
 // kMix: render modes 4, 12, 13 (1) and 14 (2, grid levels times the weight):
 // per-splat features ahead of the grid's; the
 // queue then carries a 32-bit meta word per hit (drain_mixed) in place of
-// the level count, 53 KB of LDS in all.
+// the level count, 50.4 KB of LDS in all.
 // kKT: the splats' kernel comes from p.kernel_type (1-3 possible); without
 // it the kernel is the Gaussian, and the kernel-type branch compiles out.
 // kHsh: render modes 8, 9, 10 (one 3-channel grid level) and 1, 5 (surface

@@ -2,12 +2,11 @@
 // gaussian_renderer/__init__.py:763-791 and depth_to_normal
 // (utils/point_utils.py:10-60) in one pass.
 //
-// One lane per pixel.  A pixel reads its five allmap planes and, for the
-// normal, expected depth, alpha and median of its four neighbours (cached
-// lines of the same and the two adjacent rows), and writes 36 bytes.  As
-// tensor operations this was 20 launches over 12-byte rows, two of them
-// products with a 3x3 matrix.  800x800 pixels: 163 us of kernels before,
-// 10.6 now (38 MB).
+// One lane per pixel.  A pixel reads allmap planes 0-5 and, for the normal,
+// expected depth, alpha and median of its four neighbours (cached lines of the
+// same and the two adjacent rows), and writes 36 bytes.  As tensor operations
+// this was 20 launches over 12-byte rows, two of them products with a 3x3
+// matrix.  800x800 pixels: 163 us of kernels before, 10.6 now (38 MB).
 #include "nest_internal.h"
 
 namespace nest {

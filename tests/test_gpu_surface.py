@@ -53,6 +53,37 @@ def test_surface_maps_fused(W, H, ratio):
             np.testing.assert_array_equal(o.numpy(), v.numpy(), err_msg=k)
 
 
+@pytest.mark.parametrize("ratio", [0.0, 0.3])
+def test_surface_normal_against_64_bits(ratio):
+    """The normal of the back-projected depth map in 64 bits, from the same
+    32-bit map, ray matrix and view matrix.  A point's coordinates come from
+    terms below 4 with three 32-bit roundings (7e-7); each of the two
+    differences, at least 0.04 long, errs by up to twice that, 3.6e-5 of its
+    length: 7e-5 of the normal, so 1e-4."""
+    from nest_splat.camera import look_at, view_ray_matrix
+    from nest_splat.renderer import surface_maps
+    W, H = 97, 61
+    cam = look_at((0.4, -3.0, 1.0), (0, 0, 0), 50.0, W, H)
+    a = _allmap(W, H, 9)
+    y, x = torch.meshgrid(torch.arange(H).double(), torch.arange(W).double(), indexing="ij")
+    a[1] = a[1].clamp_min(0.3)
+    a[0] = ((3 + 0.3 * torch.sin(x / 7) + 0.2 * torch.cos(y / 5)) * a[1]).float()
+    a[5] = a[0] / a[1] + 0.01
+    d = a.double()
+    depth = (1 - ratio) * d[0] / d[1] + ratio * d[5]
+    rays = torch.stack([x, y, torch.ones_like(x)], -1) @ torch.from_numpy(view_ray_matrix(cam)).double()
+    origin = np.linalg.inv(np.asarray(cam.world_view_transform, dtype=np.float64).T)[:3, 3]
+    pts = depth[..., None] * rays + torch.from_numpy(origin)
+    dy, dx = pts[2:, 1:-1] - pts[:-2, 1:-1], pts[1:-1, 2:] - pts[1:-1, :-2]
+    assert dx.norm(dim=-1).min() > 0.04 and dy.norm(dim=-1).min() > 0.04 and pts.abs().max() < 4
+    n = torch.zeros((H, W, 3), dtype=torch.float64)
+    n[1:-1, 1:-1] = torch.nn.functional.normalize(torch.cross(dy, dx, dim=-1), dim=-1)
+    out = surface_maps(cam, a.to(DEV), ratio)["surf_normal"].cpu().double()
+    err = (out - (n * d[1][..., None]).permute(2, 0, 1)).abs().max().item()
+    print(f"surf_normal max error {err:.1e}", flush=True)
+    assert err <= 1e-4
+
+
 def test_surface_maps_gradient_and_views_keep_the_general_path():
     """A map that gradients follow, and one that is not contiguous."""
     from nest_splat.camera import look_at
