@@ -853,11 +853,12 @@ constexpr uint32_t kWideSplat = 24;
 // contributor, conservative test), back to front, then every lane works
 // through its own list: exact test, blending recursion, gradients into the
 // batch's LDS sums.  A splat of kWideSplat candidates or more is taken by all
-// of them at once (lists let the lanes drift apart, which splits its sum).  Bound by the recursion's serial arithmetic and the ~15
-// LDS adds per hit.  The lockstep walk below visits every splat of the tile
-// with 18 wave sums and atomics per splat; 200k splats, SH degree 3, 800x800:
-// 2.92 ms there, 1.17 ms here (2.26 with every lane adding for itself: LDS adds
-// to one address run one after the other).
+// of them at once (lists let the lanes drift apart, which splits its sum).
+// Bound by the recursion's serial arithmetic and the ~15 LDS adds per hit (VALU
+// issue 0.60 at 2 waves a SIMD).  The lockstep walk below visits every splat of
+// the tile with 18 wave sums and atomics per splat; 200k splats, SH degree 3,
+// 800x800: 2.92 ms there, 1.17 ms here (2.26 with every lane adding for itself:
+// LDS adds to one address run one after the other).
 __global__ void __launch_bounds__(kBwdThreads) render_backward_rgb_kernel(const RenderBwdParams p) {
   __shared__ float4 srec[4][kBwdThreads];  // record chunks 0-3, the shape in place of the appearance level
   __shared__ float scut[kBwdThreads];
