@@ -990,7 +990,10 @@ static hipError_t launch_f32_tiles(const MlpParams& p, hipStream_t s) {
 
 // One 16-pixel tile per wave while that leaves at most two waves on a SIMD
 // (a 128x128 frame is 256 workgroups), two tiles sharing their weight reads
-// beyond.
+// beyond.  Calls with one / two tiles, us (12.7 is the host's part): 128 channels at
+// width 64 8,192 pixels 13.0 / 17.5, 16,384 13.3 / 17.7, 32,768 21.3 / 19.3, 49,152
+// 39.1 / 30.0, 640,000 251 / 220; 32 channels 32,768 13.0 / 12.7, 49,152 20.4 / 17.5,
+// 640,000 119 / 113; 16 at width 16 640,000 38.1 / 39.4.
 template <int NT>
 static hipError_t launch_f32(const MlpParams& p, hipStream_t s) {
   return p.N <= 32768 ? launch_f32_tiles<NT, 1>(p, s) : launch_f32_tiles<NT, 2>(p, s);
